@@ -353,7 +353,9 @@ int kmi_lattice_get_launch(const kmi_lattice* lat, int32_t* bx, int32_t* by, int
  * D2Q9 lattices without cut links or per-node faces (thermal: not F64), at least the tile
  * plus its ring on each axis, zchunks 1; the tile and a ring of as many cells as steps are
  * advanced in LDS, one work-item per cell: 1 = 28x28 two steps, 2 = 24x24 four, 3 = 56x8
- * four, 4 = 16x16 eight, 5 = 60x12 two, 6 = 8x8 four, 7 = 16x16 four, 8 = 8x8 eight.
+ * four, 4 = 16x16 eight, 5 = 60x12 two, 6 = 8x8 four, 7 = 16x16 four, 8 = 8x8 eight.  Tile 2
+ * of a lattice of at least 160,000 cells without mask, forcing or thermal populations marches
+ * strips of columns in registers instead (four steps as well).
  * Results are bit-identical to single-step launches; step counts that are not a multiple
  * of the span end with single steps. */
 int kmi_lattice_set_temporal(kmi_lattice* lat, int32_t tile, int32_t zchunks);
@@ -433,9 +435,9 @@ int kmi_batch_set_launch(kmi_batch* b, int32_t tw, int32_t th, int32_t groups, i
 int kmi_batch_get_launch(const kmi_batch* b, int32_t* tw, int32_t* th, int32_t* groups,
                          int32_t* nontemporal);
 /* Steps per launch: 1; 2 (the tile's step t+1, with a one-cell ring, kept in LDS; HBM
- * sees one read and one write per population per two steps); 3 or 4 (the tile and a
- * 3- or 4-cell ring advanced in LDS, one work-item per cell of that region; tiles of width
- * 16, 32 or 64).  Bit-identical to single steps; step counts that are not a multiple end
+ * sees one read and one write per population per two steps); 3 or 4 (strips of columns
+ * marched up the cavities, the intermediate steps in registers; tiles of width 16, 32 or 64,
+ * which the residual sums keep using).  Bit-identical to single steps; step counts that are not a multiple end
  * with two-step and single-step launches.  Chosen by kmi_batch_autotune. */
 int kmi_batch_set_temporal(kmi_batch* b, int32_t steps_per_launch);
 int kmi_batch_get_temporal(const kmi_batch* b, int32_t* steps_per_launch);

@@ -429,6 +429,16 @@ static bool tb_eligible(const kmi_lattice* L, int tile) {
   return true;
 }
 
+// Whether tile 2 (24×24, four steps) of a D2Q9 lattice runs the register march
+// (kmi_march2d.hip): no thermal populations, mask or forcing, and at least 160,000 cells.
+// Below that the march has too few waves (µs per step, tile / march, F64 periodic: 320² 4.4 /
+// 4.5, 400² 6.9 / 4.6, 512² 8.1 / 5.6, 2048² 90 / 40; F32S cavity: 320² 3.3 / 5.0, 400² 5.2 /
+// 5.0, 640² 7.6 / 6.2, 2048² 61 / 23).
+static bool march_applies(const kmi_lattice* L) {
+  return L->Q == 9 && L->tb_tile == 2 && !L->desc.thermal && !L->mask && L->desc.forcing == KMI_FORCE_NONE &&
+         L->ncells >= 160000;
+}
+
 // Steps advanced by one launch.
 static int launch_span(const kmi_lattice* L) {
   if (!L->tb_tile || !tb_eligible(L, L->tb_tile)) return 1;
@@ -459,13 +469,16 @@ static int launch_one(kmi_lattice* L, hipStream_t s, bool multi = false) {
                          L->order_key[1] == L->tb_zchunks
                      ? L->order
                      : nullptr;
-  hipError_t e =
-      multi ? (L->Q == 9 ? launch_step_tb2d(L->desc.storage, L->desc.collision, L->tb_tile,
-                                            L->desc.thermal != 0, a, s)
-                         : launch_step2(L->desc.storage, L->desc.collision, L->tb_tile, L->tb_zchunks,
-                                        L->nts != 0, L->bnd, a, s))
-            : launch_step(L->Q, L->desc.storage, L->desc.collision, L->desc.thermal != 0, L->bnd,
-                          L->nts != 0, a, L->grid, L->block, s);
+  hipError_t e;
+  if (!multi)
+    e = launch_step(L->Q, L->desc.storage, L->desc.collision, L->desc.thermal != 0, L->bnd, L->nts != 0, a,
+                    L->grid, L->block, s);
+  else if (L->Q == 19)
+    e = launch_step2(L->desc.storage, L->desc.collision, L->tb_tile, L->tb_zchunks, L->nts != 0, L->bnd, a, s);
+  else if (march_applies(L))
+    e = launch_march2d(L->desc.storage, L->desc.collision, a, s);
+  else
+    e = launch_step_tb2d(L->desc.storage, L->desc.collision, L->tb_tile, L->desc.thermal != 0, a, s);
   if (e != hipSuccess) return hip_fail(L->ctx, e, "step kernel launch");
   L->cur ^= 1;
   return KMI_OK;

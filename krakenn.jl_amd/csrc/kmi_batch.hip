@@ -13,10 +13,12 @@
 #include <cmath>
 #include <cstring>
 #include <new>
+#include <utility>
 #include <vector>
 
 #include "kmi_cell.h"
 #include "kmi_internal.h"
+#include "kmi_march2d.h"
 
 namespace kmi {
 
@@ -180,74 +182,63 @@ __global__ void __launch_bounds__(256) k_batch_step2(const BatchArgs a) {
   }
 }
 
-// K steps per launch (K = 3 or 4) over the same tile slots: the tile and a K-cell ring are
-// loaded into LDS with one work-item per cell of that region ((tw+2K)(th+2K) ≤ 1024), then
-// advanced K steps in place (step s updates the region less s cells on each side: read,
-// barrier, write back in the storage rounding, barrier); the tile's t+K populations go to
-// HBM.  Bit-identical to K single steps.  Dynamic LDS: 9 · (tw+2K)(th+2K) reals.
-template <int ST, int COLL, int K>
-__global__ void __launch_bounds__(1024) k_batch_stepK(const BatchArgs a) {
-  using S = Store<ST>;
-  using E = typename S::elem;
-  using R = typename S::real;
-  R* const L = reinterpret_cast<R*>(kmi_batch_lds);
-  const int tw = a.tw, th = 256 / a.tw;
-  const int ew = tw + 2 * K, eh = th + 2 * K, ne = ew * eh;
-  const int e = threadIdx.x;  // one work-item per region cell (blockDim.x == ne)
-  const int ex = e % ew, ey = e / ew;
-  for (int t = blockIdx.x; t < a.nslots; t += gridDim.x) {
-    const int c = a.slots[3 * t];  // uniform over the work-group
-    if (c < 0) continue;
-    const CavRec cv = a.cav[c];
-    const int n = cv.n;
-    const int i = a.slots[3 * t + 1] - K + ex, j = a.slots[3 * t + 2] - K + ey;
-    const bool in = i >= 0 && j >= 0 && i < n && j < n;
-    const unsigned P = unsigned(n) * unsigned(n);
-    const E* __restrict__ src = static_cast<const E*>(a.fi) + cv.foff;
-    E* __restrict__ dst = static_cast<E*>(a.fo) + cv.foff;
-    if (in) {
-      const unsigned self = unsigned(i + n * j);
-      sfor<9>([&](auto qc) {
-        constexpr int q = decltype(qc)::value;
-        L[q * ne + e] = S::ld(src, self + unsigned(q) * P);
-      });
+// K steps per launch (K = 3 or 4): the register march of kmi_march2d.h, one wave per piece
+// (cavity, columns [x0, x1), rows [y0, y1)) of a table the host lays out (batch_build_pieces).
+// Bit-identical to K single steps.  256 cavities of 64–512 cells a side, F32S MRT: 172 (K = 3)
+// and 221 GLUPS (K = 4) where a kernel that advanced each tile and its K-cell ring in LDS ran
+// 122 and 117; 256 of 128²: 167 and 204 against 129 and 119.  The two-step tile kernel above
+// (124 and 114 GLUPS) stays for two steps: marching K = 2 levels runs 89–121.
+struct MarchPiece {
+  int cav;        // −1: padding
+  int x0x1, y0y1;  // first and one past the last column / row, 16 bits each
+  int pad;
+};
+
+template <int ST, int COLL>
+struct CavityDom {
+  using E = typename Store<ST>::elem;
+  using R = typename Store<ST>::real;
+  static constexpr bool SH = Store<ST>::shifted;
+  static constexpr bool perx = false, pery = false;
+  const BatchArgs& a;
+  const CavRec cv;
+  int nx, ny;
+  KMI_DEV CavityDom(const BatchArgs& args, const CavRec& c) : a(args), cv(c), nx(c.n), ny(c.n) {}
+  KMI_DEV const E* src(int q) const { return static_cast<const E*>(a.fi) + cv.foff + (long long)q * nx * nx; }
+  KMI_DEV E* dst(int q) const { return static_cast<E*>(a.fo) + cv.foff + (long long)q * nx * nx; }
+  template <int q, bool ROWS>
+  KMI_DEV R ladd(R v, bool, bool, bool, bool wyp) const {
+    if constexpr (ROWS && Lat<9>::cy[q] < 0) {
+      if (wyp && a.lid == KMI_FACE_MOVING_WALL)
+        v = v + R(six_w(Lat<9>::w[q])) * R(1.0) * cdotu<Lat<9>::cx[q], Lat<9>::cy[q], 0>(R(a.u_lid), R(0.0), R(0.0));
     }
-    __syncthreads();
-    R fr[9];
-    for (int s = 1; s <= K; ++s) {
-      const bool valid = in && ex >= s && ex < ew - s && ey >= s && ey < eh - s;
-      if (valid) {
-        R fp[9];
-        cavity_pull(a, n, i, j, unsigned(e), unsigned(ew), unsigned(ne), fp,
-                    [&](unsigned off) { return L[off]; });
-        cavity_collide<ST, COLL>(a, cv, n, j, fp, fr);
-      }
-      if (s == K) break;
-      __syncthreads();  // every step-s read of L is done
-      if (valid) {
-        sfor<9>([&](auto qc) {
-          constexpr int q = decltype(qc)::value;
-          L[q * ne + e] = storage_round<ST>(fr[q]);
-        });
-      }
-      __syncthreads();
-    }
-    if (in && ex >= K && ex < K + tw && ey >= K && ey < K + th) {
-      const unsigned self = unsigned(i + n * j);
-      sfor<9>([&](auto qc) {
-        constexpr int q = decltype(qc)::value;
-        S::template st<false>(dst, self + unsigned(q) * P, fr[q]);
-      });
-    }
-    __syncthreads();  // the next slot's load overwrites LDS
+    return v;
   }
+  template <bool ROWS>
+  KMI_DEV void closures(R (&fp)[9], int, int j) const {
+    if (ROWS && a.lid == KMI_FACE_ZOUHE_VELOCITY && j == ny - 1) zh_north<SH>(fp, R(a.u_lid));
+  }
+  KMI_DEV void collide(const R (&fp)[9], R (&fo)[9]) const {
+    if constexpr (COLL == KMI_BGK) collide_bgk<9, SH>(fp, fo, R(cv.om));
+    else if constexpr (COLL == KMI_TRT) collide_trt<9, SH>(fp, fo, R(cv.om), R(cv.sm));
+    else collide_mrt<SH>(fp, fo, R(a.s_e), R(a.s_eps), R(a.s_q), R(cv.om));
+  }
+};
+
+template <int ST, int COLL, int K>
+__global__ void __launch_bounds__(256, (march_waves<ST, K>()))
+    k_batch_march(const BatchArgs a, const MarchPiece* __restrict__ pieces) {
+  const int wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6));
+  const MarchPiece p = pieces[blockIdx.x * 4 + wave];
+  if (p.cav < 0) return;
+  const CavityDom<ST, COLL> d(a, a.cav[p.cav]);
+  const int xs = p.x0x1 & 0xffff, xe = p.x0x1 >> 16, y0 = p.y0y1 & 0xffff, y1 = p.y0y1 >> 16;
+  if (march_inner(d.nx, false, K, xs, xe)) march2d<ST, K, false>(d, xs, xe, y0, y1);
+  else march2d<ST, K, true>(d, xs, xe, y0, y1);
 }
 
-// Work-items of a K-step region for tile width tw (0: the region exceeds 1024).
-KMI_HD int stepK_region(int tw, int K) {
-  const int r = (tw + 2 * K) * (256 / tw + 2 * K);
-  return r <= 1024 ? r : 0;
-}
+// Tile widths that 3 or 4 steps per launch take (the tiles still carry the residual).
+static bool stepK_tile(int tw, int K) { return (tw + 2 * K) * (256 / tw + 2 * K) <= 1024; }
 
 // Velocity of a cell from the stored populations, FP64 (compute_macroscopic_2d order).
 template <int ST>
@@ -439,25 +430,23 @@ static hipError_t launch_batch_step2(int st, int coll, bool nts, const BatchArgs
   return hipGetLastError();
 }
 
-static hipError_t launch_batch_stepK(int st, int coll, int K, const BatchArgs& a, int groups, hipStream_t s) {
-  const int ne = stepK_region(a.tw, K);
-  if (ne == 0) return hipErrorInvalidValue;
-  const dim3 g(static_cast<unsigned>(groups)), b(static_cast<unsigned>(ne));
-#define KMI_BATCH_COLLK(ST)                                                                      \
+static hipError_t launch_batch_march(int st, int coll, int K, const BatchArgs& a, const MarchPiece* pieces,
+                                     int npieces, hipStream_t s) {
+  const dim3 g(static_cast<unsigned>(npieces / 4)), b(256);
+#define KMI_BATCH_MARCH_K(ST, COLL)                                                              \
   {                                                                                             \
-    const size_t sh = size_t(9) * ne * sizeof(typename Store<ST>::real);                        \
-    if (K == 3) {                                                                               \
-      if (coll == KMI_BGK) hipLaunchKernelGGL((k_batch_stepK<ST, KMI_BGK, 3>), g, b, sh, s, a); \
-      else if (coll == KMI_TRT) hipLaunchKernelGGL((k_batch_stepK<ST, KMI_TRT, 3>), g, b, sh, s, a); \
-      else hipLaunchKernelGGL((k_batch_stepK<ST, KMI_MRT, 3>), g, b, sh, s, a);                 \
-    } else {                                                                                    \
-      if (coll == KMI_BGK) hipLaunchKernelGGL((k_batch_stepK<ST, KMI_BGK, 4>), g, b, sh, s, a); \
-      else if (coll == KMI_TRT) hipLaunchKernelGGL((k_batch_stepK<ST, KMI_TRT, 4>), g, b, sh, s, a); \
-      else hipLaunchKernelGGL((k_batch_stepK<ST, KMI_MRT, 4>), g, b, sh, s, a);                 \
-    }                                                                                           \
+    if (K == 3) hipLaunchKernelGGL((k_batch_march<ST, COLL, 3>), g, b, 0, s, a, pieces);        \
+    else hipLaunchKernelGGL((k_batch_march<ST, COLL, 4>), g, b, 0, s, a, pieces);               \
   }
-  KMI_BATCH_ST(st, KMI_BATCH_COLLK(ST));
-#undef KMI_BATCH_COLLK
+#define KMI_BATCH_MARCH(ST)                              \
+  {                                                     \
+    if (coll == KMI_BGK) KMI_BATCH_MARCH_K(ST, KMI_BGK) \
+    else if (coll == KMI_TRT) KMI_BATCH_MARCH_K(ST, KMI_TRT) \
+    else KMI_BATCH_MARCH_K(ST, KMI_MRT)                 \
+  }
+  KMI_BATCH_ST(st, KMI_BATCH_MARCH(ST));
+#undef KMI_BATCH_MARCH
+#undef KMI_BATCH_MARCH_K
   return hipGetLastError();
 }
 
@@ -491,13 +480,16 @@ struct kmi_batch {
   int cur = 0;
   // tiles
   int tw = 64, th = 4, groups = 0, nts = 0;
-  int span = 1;  // steps per launch: 1, 2 (k_batch_step2), 3 or 4 (k_batch_stepK)
+  int span = 1;  // steps per launch: 1, 2 (k_batch_step2), 3 or 4 (k_batch_march)
   bool tiles_dirty = true;
   int nslots = 0;
   int* slots_d = nullptr;
   size_t slots_cap = 0;
   int* cav_slots_d = nullptr;
   size_t cav_slots_cap = 0;
+  int npieces = 0;  // pieces of the register march (span 3 or 4), a multiple of 4
+  MarchPiece* pieces_d = nullptr;
+  size_t pieces_cap = 0;
   int* cav_range_d = nullptr;
   int* active_d = nullptr;
   double* uprev = nullptr;
@@ -525,6 +517,54 @@ static int batch_groups(const kmi_batch* B) {
   int g = B->groups > 0 ? std::min(B->groups, B->nslots) : B->nslots;
   g = ((g + 7) / 8) * 8;  // multiple of 8: slot s keeps running on XCD s mod 8
   return std::max(g, 8);
+}
+
+// Pieces of the register march, cavity-major with neighbouring strips side by side, then
+// permuted by work-groups of four so that each XCD (work-group b runs on XCD b mod 8) owns one
+// contiguous run.
+static void batch_build_pieces(kmi_batch* B, std::vector<MarchPiece>& out) {
+  out.clear();
+  B->npieces = 0;
+  if (B->span < 3) return;
+  std::vector<std::pair<int, int>> sides;  // (side, running cavities)
+  for (int cv = 0; cv < B->ncav; ++cv) {
+    if (B->status[cv] != KMI_CAV_RUNNING) continue;
+    size_t k = 0;
+    while (k < sides.size() && sides[k].first != B->n[cv]) ++k;
+    if (k == sides.size()) sides.emplace_back(B->n[cv], 0);
+    ++sides[k].second;
+  }
+  auto count = [&](int r) {
+    long long c = 0;
+    for (const auto& [n, cavities] : sides)
+      c += (long long)cavities * march_strips(n, B->span, false).m * ((n + r - 1) / r);
+    return c;
+  };
+  // Few enough pieces to be resident at once: march_rows.  More of them: short pieces, whose
+  // neighbours stay close together (256 cavities of 64–512 a side, F32S MRT, four steps:
+  // 206 / 221 / 212 / 202 GLUPS at 8 / 12 / 19 / 32 rows; three steps: 172 / 164 / 150 / 144).
+  const int resident = B->esize == sizeof(double) ? 2 : (B->span >= 4 ? 3 : 4);
+  int rows = march_rows(128, resident, count);
+  if (count(rows) > 1024LL * resident) rows = B->span >= 4 ? 12 : 8;
+  std::vector<MarchPiece> p;
+  for (int cv = 0; cv < B->ncav; ++cv) {
+    if (B->status[cv] != KMI_CAV_RUNNING) continue;
+    const int n = B->n[cv];
+    const MarchStrips st = march_strips(n, B->span, false);
+    const int chunks = (n + rows - 1) / rows;
+    for (int ch = 0; ch < chunks; ++ch)
+      for (int k = 0; k < st.m; ++k)
+        p.push_back(MarchPiece{cv, st.start(k) | (st.start(k + 1) << 16),
+                               int((long long)n * ch / chunks) | (int((long long)n * (ch + 1) / chunks) << 16), 0});
+  }
+  const int groups = (int(p.size()) + 3) / 4, per_xcd = (groups + 7) / 8;
+  out.assign(size_t(32) * per_xcd, MarchPiece{-1, 0, 0, 0});
+  for (int b = 0; b < 8 * per_xcd; ++b) {
+    const int t = (b % 8) * per_xcd + b / 8;
+    for (int w = 0; w < 4; ++w)
+      if (size_t(4 * t + w) < p.size()) out[size_t(4 * b + w)] = p[size_t(4 * t + w)];
+  }
+  B->npieces = int(out.size());
 }
 
 // Cavity-major tile order, then slot permutation so XCD x owns run x of that order.
@@ -577,6 +617,12 @@ static int batch_build_tiles(kmi_batch* B) {
   KMI_HIP(c, grow((void**)&B->slots_d, B->slots_cap, slots.size() * sizeof(int)));
   KMI_HIP(c, grow((void**)&B->cav_slots_d, B->cav_slots_cap, cav_slots.size() * sizeof(int)));
   KMI_HIP(c, grow((void**)&B->partials, B->partials_cap, size_t(4) * B->nslots * sizeof(double)));
+  std::vector<MarchPiece> pieces;
+  batch_build_pieces(B, pieces);
+  if (!pieces.empty()) {
+    KMI_HIP(c, grow((void**)&B->pieces_d, B->pieces_cap, pieces.size() * sizeof(MarchPiece)));
+    KMI_HIP(c, hipMemcpy(B->pieces_d, pieces.data(), pieces.size() * sizeof(MarchPiece), hipMemcpyHostToDevice));
+  }
   KMI_HIP(c, hipMemcpy(B->slots_d, slots.data(), slots.size() * sizeof(int), hipMemcpyHostToDevice));
   KMI_HIP(c, hipMemcpy(B->cav_slots_d, cav_slots.data(), cav_slots.size() * sizeof(int), hipMemcpyHostToDevice));
   KMI_HIP(c, hipMemcpy(B->cav_range_d, range.data(), range.size() * sizeof(int), hipMemcpyHostToDevice));
@@ -623,9 +669,10 @@ static int batch_launch_step2(kmi_batch* B, hipStream_t s) {
   return KMI_OK;
 }
 
-static int batch_launch_stepK(kmi_batch* B, hipStream_t s) {
+static int batch_launch_march(kmi_batch* B, hipStream_t s) {
   BatchArgs a = batch_args(B);
-  hipError_t e = launch_batch_stepK(B->desc.storage, B->desc.collision, B->span, a, batch_groups(B), s);
+  hipError_t e =
+      launch_batch_march(B->desc.storage, B->desc.collision, B->span, a, B->pieces_d, B->npieces, s);
   if (e != hipSuccess) return hip_fail(B->ctx, e, "batch multi-step launch");
   B->cur ^= 1;
   return KMI_OK;
@@ -635,7 +682,7 @@ static int batch_launch_stepK(kmi_batch* B, hipStream_t s) {
 static int batch_launch_n(kmi_batch* B, int64_t n, hipStream_t s) {
   if (B->span >= 3)
     for (; n >= B->span; n -= B->span)
-      if (int rc = batch_launch_stepK(B, s)) return rc;
+      if (int rc = batch_launch_march(B, s)) return rc;
   if (B->span >= 2)
     for (; n >= 2; n -= 2)
       if (int rc = batch_launch_step2(B, s)) return rc;
@@ -755,7 +802,7 @@ int kmi_batch_destroy(kmi_batch* B) {
   (void)hipStreamSynchronize(B->ctx->stream);
   batch_drop_graphs(B);
   void* ptrs[] = {B->f[0], B->f[1], B->cav_d, B->slots_d, B->cav_slots_d, B->cav_range_d,
-                  B->active_d, B->uprev, B->partials, B->resid_d};
+                  B->pieces_d, B->active_d, B->uprev, B->partials, B->resid_d};
   for (void* p : ptrs)
     if (p) (void)hipFree(p);
   for (auto ev : B->ev)
@@ -1023,7 +1070,7 @@ int kmi_batch_set_launch(kmi_batch* B, int32_t tw, int32_t th, int32_t groups, i
   if (!B) return fail(nullptr, KMI_ERR_ARG, "batch is NULL");
   if (!((tw == 16 || tw == 32 || tw == 64 || tw == 128 || tw == 256) && tw * th == 256) || groups < 0)
     return fail(B->ctx, KMI_ERR_ARG, "kmi_batch_set_launch: tiles of tw x th = 256 cells, tw in {16,32,64,128,256}");
-  if (B->span >= 3 && stepK_region(tw, B->span) == 0)
+  if (B->span >= 3 && !stepK_tile(tw, B->span))
     return fail(B->ctx, KMI_ERR_ARG, "kmi_batch_set_launch: tile too wide for the current steps per launch");
   KMI_HIP(B->ctx, hipSetDevice(B->ctx->device));
   KMI_HIP(B->ctx, hipStreamSynchronize(B->ctx->stream));
@@ -1040,12 +1087,13 @@ int kmi_batch_set_temporal(kmi_batch* B, int32_t steps_per_launch) {
   if (!B) return fail(nullptr, KMI_ERR_ARG, "batch is NULL");
   if (steps_per_launch < 1 || steps_per_launch > 4)
     return fail(B->ctx, KMI_ERR_ARG, "kmi_batch_set_temporal: steps per launch must be 1, 2, 3 or 4");
-  if (steps_per_launch >= 3 && stepK_region(B->tw, steps_per_launch) == 0)
+  if (steps_per_launch >= 3 && !stepK_tile(B->tw, steps_per_launch))
     return fail(B->ctx, KMI_ERR_ARG,
                 "kmi_batch_set_temporal: 3 or 4 steps per launch need tiles of width 16, 32 or 64");
   KMI_HIP(B->ctx, hipSetDevice(B->ctx->device));
   KMI_HIP(B->ctx, hipStreamSynchronize(B->ctx->stream));
   B->span = steps_per_launch;
+  B->tiles_dirty = true;
   batch_drop_graphs(B);
   return KMI_OK;
 }
@@ -1090,7 +1138,8 @@ int kmi_batch_autotune(kmi_batch* B, int64_t steps_per_trial, double* best_ms) {
         B->groups = g;
         B->nts = nt & 1;
         B->span = 1 + (nt >> 1);
-        if (B->span >= 3 && (B->nts || stepK_region(B->tw, B->span) == 0)) continue;  // K-step stores are plain
+        // the register march depends on neither tile, groups nor store policy: timed once
+        if (B->span >= 3 && (B->nts || g != 0 || B->tw != 64)) continue;
         if (batch_build_tiles(B) != KMI_OK) { e = hipErrorUnknown; break; }
         if (g > 0 && g >= B->nslots) continue;  // same as one group per slot
         if (batch_launch_n(B, B->span, x->stream) != KMI_OK) { e = hipErrorUnknown; break; }
