@@ -56,6 +56,14 @@ KMI_DEV int wrap(int v, int n) { return v < 0 ? v + n : (v >= n ? v - n : v); }
 // other tiles (any wall, Zou–He face or solid cell), 3 for those tiles when the lattice has
 // no solid mask and its x and y faces are periodic or resting walls (x–y walls bounce links
 // back with no Ladd term and carry no Zou–He closure; the z faces are handled as in mode 1).
+// 6 and 7 are the iterations of modes 1 and 3 whose planes all lie off the z walls (or whose
+// z axis is periodic): no face in reach, and resting x–y walls only.  Most iterations are
+// such, and the z faces' bounce, Ladd terms and closures cost the loop a third of its
+// instructions and, in FP64, the registers that keep it from spilling.
+constexpr bool ring(int m) { return m == 2 || m == 3 || m == 7; }  // x–y walls in reach
+constexpr bool zfaces(int m) { return m == 1 || m == 2 || m == 3; }  // z faces in reach
+constexpr int off_z(int m) { return m == 1 ? 6 : m == 3 ? 7 : m; }   // the mode off the z faces
+
 // Whether a cell's neighbour exists along each axis direction — a periodic axis always wraps;
 // a wall face has none beyond it.
 struct Nbr {
@@ -64,7 +72,7 @@ struct Nbr {
 template <int BND>
 KMI_DEV Nbr nbr(const StepArgs& a, int gx, int gy, int gz) {
   Nbr n;
-  if constexpr (BND == 1) {
+  if constexpr (!ring(BND)) {
     n.xm = n.xp = n.ym = n.yp = true;
   } else {
     n.xm = a.per[0] || gx > 0;
@@ -72,8 +80,8 @@ KMI_DEV Nbr nbr(const StepArgs& a, int gx, int gy, int gz) {
     n.ym = a.per[1] || gy > 0;
     n.yp = a.per[1] || gy < a.ny - 1;
   }
-  n.zm = a.per[2] || gz > 0;
-  n.zp = a.per[2] || gz < a.nz - 1;
+  n.zm = !zfaces(BND) || a.per[2] || gz > 0;
+  n.zp = !zfaces(BND) || a.per[2] || gz < a.nz - 1;
   return n;
 }
 
@@ -102,6 +110,18 @@ KMI_DEV R ladd(R v, const StepArgs& a, const Nbr& n) {
   if (cz > 0 && !n.zm) add(KMI_BOTTOM);
   if (cz < 0 && !n.zp) add(KMI_TOP);
   return v;
+}
+
+// The Ladd terms of every bounced link of a cell (lattices with a moving face only).
+template <int BND, class R>
+KMI_DEV void ladd_all(R (&f)[19], const StepArgs& a, const Nbr& n) {
+  if constexpr (!zfaces(BND)) return;
+  if (!a.any_moving) return;
+  sfor<18>([&](auto qc) {
+    constexpr int q = decltype(qc)::value + 1;
+    if constexpr (BND == 2 || Lat<19>::cz[q] != 0)  // modes 1 and 3: only z faces move
+      if (!src_ok<q>(n)) f[q] = ladd<q, BND>(f[q], a, n);
+  });
 }
 
 // Element at byte offset `off` of a population plane.  Plane bases are uniform (scalar
@@ -218,23 +238,35 @@ KMI_DEV void pull_lds(R (&fp)[19], const R* A, const R* Bs, const R* Cs, const R
     constexpr int q = decltype(qc)::value;
     constexpr int cx = Lat<19>::cx[q], cy = Lat<19>::cy[q], cz = Lat<19>::cz[q];
     constexpr int n = tb::group_index(q), o = Lat<19>::opp[q], no = tb::group_index(o);
-    bool ok = true;
-    if constexpr (BND) ok = tb::src_ok<q>(nb);
-    if (ok) {
-      const int e = (ey - cy) * EXp + (ex - cx);
-      if constexpr (cz == 0) fp[q] = A[n * NEp + e];
-      else if constexpr (cz > 0) fp[q] = Bs[n * NEp + e];
-      else fp[q] = Cs[n * NEp + e];
-    } else if constexpr (BND) {
-      R v;
-      if constexpr (cz == 0) v = A[no * NEp + own];
-      else if constexpr (cz > 0) v = Co[no * NEp + own];  // opp(q) has c_z = −1
-      else v = Bo[no * NEp + own];
-      if constexpr (q != 0)
-        if (a.any_moving) v = tb::ladd<q, BND>(v, a, nb);
-      fp[q] = v;
+    const int e = (ey - cy) * EXp + (ex - cx);
+    const R* src = (cz == 0 ? A : cz > 0 ? Bs : Cs) + n * NEp + e;
+    if constexpr (BND && q != 0) {
+      // one read at a selected address: written as branches, the bounced links put a divergent
+      // branch on every link (run_cavity_3d's cube, F32S 256³ on 64×8 tiles, µs per step:
+      // branches 382, selects 298, selects with the iterations off the z faces apart 279;
+      // F64 128³ on 32×8 tiles: 117, 97, 88)
+      const R* back = (cz == 0 ? A : cz > 0 ? Co : Bo) + no * NEp + own;
+      src = tb::src_ok<q>(nb) ? src : back;
     }
+    fp[q] = *src;
   });
+  if constexpr (BND) tb::ladd_all<BND>(fp, a, nb);
+}
+
+// Runs iterate(s, mode) over planes lo … hi.  An iteration of a SPAN-step march evaluates
+// planes s, s − 1, … s − SPAN + 1 and may pull plane s + 1; where all of them lie off the z
+// faces it runs in the mode without them.
+template <int BND, int SPAN, class F>
+KMI_DEV void march_planes(const StepArgs& a, int lo, int hi, int nz, F&& iterate) {
+  constexpr std::integral_constant<int, BND> edge{};
+  constexpr std::integral_constant<int, tb::off_z(BND)> main{};
+  int s = lo;
+  if constexpr (tb::off_z(BND) != BND) {
+    const int first = a.per[2] ? lo : SPAN, last = a.per[2] ? hi : nz - 3;
+    for (; s < first && s <= hi; ++s) iterate(s, edge);
+    for (; s <= last && s <= hi; ++s) iterate(s, main);
+  }
+  for (; s <= hi; ++s) iterate(s, edge);
 }
 
 // The two-step march of one column tile (tx, ty) over z-range zc, LDS at `lds`.
@@ -273,20 +305,24 @@ KMI_DEV void march2(const StepArgs& a, int zlen, int tx, int ty, int zc, typenam
   // Ladd term of a moving wall); extended cells beyond a wall are never read and skipped.
   constexpr bool kPrefetch = sizeof(R) == 4 && (NT <= 512 || EPT == 1);
   R nxt[EPT][19];
-  auto inside = [&](int s, int e) {
-    if constexpr (BND == 0) return true;
-    if constexpr (BND == 1) return a.per[2] || (s >= 0 && s < nz);
-    const int ux = x0 - 1 + e % EX, uy = y0 - 1 + e / EX;
-    return (a.per[0] || (ux >= 0 && ux < nx)) && (a.per[1] || (uy >= 0 && uy < ny)) &&
-           (a.per[2] || (s >= 0 && s < nz));
+  auto inside = [&](int s, int e, auto mc) {
+    constexpr int M = decltype(mc)::value;
+    bool in = true;
+    if constexpr (tb::ring(M)) {
+      const int ux = x0 - 1 + e % EX, uy = y0 - 1 + e / EX;
+      in = (a.per[0] || (ux >= 0 && ux < nx)) && (a.per[1] || (uy >= 0 && uy < ny));
+    }
+    if constexpr (tb::zfaces(M)) in = in && (a.per[2] || (s >= 0 && s < nz));
+    return in;
   };
-  auto pull_plane = [&](int s) {
+  auto pull_plane = [&](int s, auto mc) {
+    constexpr int M = decltype(mc)::value;
     const int zs = tb::wrap(s, nz);
     const int zm = tb::wrap(zs - 1, nz), zp = tb::wrap(zs + 1, nz);
 #pragma unroll
     for (int r = 0; r < EPT; ++r) {
       const int e = tid + r * NT;
-      if (e < NE && inside(s, e)) {
+      if (e < NE && inside(s, e, mc)) {
         const int ex = e % EX, ey = e / EX;
         const int gx = tb::wrap(x0 - 1 + ex, nx), gy = tb::wrap(y0 - 1 + ey, ny);
         const int xm = tb::wrap(gx - 1, nx), xp = tb::wrap(gx + 1, nx);
@@ -295,48 +331,49 @@ KMI_DEV void march2(const StepArgs& a, int zlen, int tx, int ty, int zc, typenam
         const unsigned bx[3] = {unsigned(xm) * ES, unsigned(gx) * ES, unsigned(xp) * ES};
         const int yy[3] = {ym, gy, yp}, zz[3] = {zm, zs, zp};
         tb::Nbr nb{};
-        if constexpr (BND) nb = tb::nbr<BND>(a, gx, gy, zs);
+        if constexpr (M != 0) nb = tb::nbr<M>(a, gx, gy, zs);
         const unsigned own = (unsigned(gx) + unsigned(nx) * unsigned(gy + ny * zs)) * ES;
         sfor<19>([&](auto qc) {
           constexpr int q = decltype(qc)::value;
           constexpr int cx = Lat<19>::cx[q], cy = Lat<19>::cy[q], cz = Lat<19>::cz[q];
-          bool ok = true;
-          if constexpr (BND) ok = tb::src_ok<q>(nb);
-          if (ok) {
-            const unsigned row = unsigned(nx) * unsigned(yy[1 - cy] + ny * zz[1 - cz]) * ES;
-            nxt[r][q] = Pops<ST>::ld(&tb::at(fi + q * P, row + bx[1 - cx]));
-          } else if constexpr (BND) {
-            R v = Pops<ST>::ld(&tb::at(fi + Lat<19>::opp[q] * P, own));
-            if constexpr (q != 0)
-              if (a.any_moving) v = tb::ladd<q, BND>(v, a, nb);
-            nxt[r][q] = v;
+          const unsigned row = unsigned(nx) * unsigned(yy[1 - cy] + ny * zz[1 - cz]) * ES;
+          const E* plane = fi + q * P;
+          unsigned off = row + bx[1 - cx];
+          if constexpr (M != 0 && q != 0) {
+            const bool ok = tb::src_ok<q>(nb);
+            plane = ok ? plane : fi + Lat<19>::opp[q] * P;
+            off = ok ? off : own;
           }
+          nxt[r][q] = Pops<ST>::ld(&tb::at(plane, off));
         });
       }
     }
   };
-  if constexpr (kPrefetch) pull_plane(z0 - 1);
+  if constexpr (kPrefetch) pull_plane(z0 - 1, std::integral_constant<int, BND>{});
 
-  for (int s = z0 - 1; s <= z1; ++s) {
+  // One plane of the march; M: the mode of its cells (BND, or its form off the z faces).
+  auto iterate = [&](int s, auto mc) {
+    constexpr int M = decltype(mc)::value;
     const int u = s + 3;  // non-negative plane counter for the LDS ring slot
     R* const Cw = C + (BND ? (u & 1) : 0) * 5 * NE;
     // ---- phase 1: t+1 on plane s, extended tile ----
-    if constexpr (!kPrefetch) pull_plane(s);
+    if constexpr (!kPrefetch) pull_plane(s, mc);
     R cur[EPT][19];
 #pragma unroll
     for (int r = 0; r < EPT; ++r)
 #pragma unroll
       for (int q = 0; q < 19; ++q) cur[r][q] = nxt[r][q];
     if constexpr (kPrefetch)
-      if (s < z1) pull_plane(s + 1);
+      if (s < z1) pull_plane(s + 1, mc);
     R keep0[EPT][9], keepp[EPT][5];
 #pragma unroll
     for (int r = 0; r < EPT; ++r) {
       const int e = tid + r * NT;
-      if (e < NE && inside(s, e)) {
+      if (e < NE && inside(s, e, mc)) {
         R fn[19];
-        update19<ST, COLL, BND>(cur[r], fn, a, tb::wrap(x0 - 1 + e % EX, nx), tb::wrap(y0 - 1 + e / EX, ny),
-                                tb::wrap(s, nz));
+        const int gx = tb::wrap(x0 - 1 + e % EX, nx), gy = tb::wrap(y0 - 1 + e / EX, ny), gz = tb::wrap(s, nz);
+        if constexpr (M != 0) tb::ladd_all<M>(cur[r], a, tb::nbr<M>(a, gx, gy, gz));
+        update19<ST, COLL, M>(cur[r], fn, a, gx, gy, gz);
         sfor<19>([&](auto qc) {
           constexpr int q = decltype(qc)::value;
           constexpr int cz = Lat<19>::cz[q];
@@ -356,7 +393,7 @@ KMI_DEV void march2(const StepArgs& a, int zlen, int tx, int ty, int zc, typenam
       const R* const Co = C + (BND ? ((u - 1) & 1) : 0) * 5 * NE;  // c_z = −1 of plane s−1 (own)
       const int ix = tid % TX, iy = tid / TX;
       tb::Nbr nb{};
-      if constexpr (BND) nb = tb::nbr<BND>(a, x0 + ix, y0 + iy, s - 1);
+      if constexpr (M != 0) nb = tb::nbr<M>(a, x0 + ix, y0 + iy, s - 1);
       R fp[19], fn[19];
       if constexpr (BND == 0) {
         // the periodic pull written out: through pull_lds the allocator keeps 1–4 more
@@ -372,9 +409,9 @@ KMI_DEV void march2(const StepArgs& a, int zlen, int tx, int ty, int zc, typenam
           else fp[q] = Cw[n * NE + e];
         });
       } else {
-        pull_lds<BND>(fp, A, Br, Cw, Bo, Co, NE, EX, ix + 1, iy + 1, a, nb);
+        pull_lds<M>(fp, A, Br, Cw, Bo, Co, NE, EX, ix + 1, iy + 1, a, nb);
       }
-      update19<ST, COLL, BND>(fp, fn, a, x0 + ix, y0 + iy, s - 1);
+      update19<ST, COLL, M>(fp, fn, a, x0 + ix, y0 + iy, s - 1);
       const unsigned cell = (unsigned(x0 + ix) + unsigned(nx) * unsigned(y0 + iy + ny * (s - 1))) * ES;
       sfor<19>([&](auto qc) {
         constexpr int q = decltype(qc)::value;
@@ -388,7 +425,7 @@ KMI_DEV void march2(const StepArgs& a, int zlen, int tx, int ty, int zc, typenam
 #pragma unroll
       for (int r = 0; r < EPT; ++r) {
         const int e = tid + r * NT;
-        if (e < NE && inside(s, e)) {
+        if (e < NE && inside(s, e, mc)) {
 #pragma unroll
           for (int n = 0; n < 9; ++n) A[n * NE + e] = keep0[r][n];
 #pragma unroll
@@ -396,7 +433,8 @@ KMI_DEV void march2(const StepArgs& a, int zlen, int tx, int ty, int zc, typenam
         }
       }
     }
-  }
+  };
+  march_planes<BND, 2>(a, z0 - 1, z1, nz, iterate);
 }
 
 // Grid: one work-group per (column tile, z-range), padded to a multiple of 8.  Work-group
@@ -499,21 +537,23 @@ KMI_DEV void march3(const StepArgs& a, int zlen, int tx, int ty, int zc, typenam
   const int tid = threadIdx.x;
 
   // cell (ux, uy) of plane s lies in the domain (walled lattices; periodic axes always)
-  auto inside = [&](int ux, int uy, int s) {
-    if constexpr (BND == 0) return true;
-    if constexpr (BND == 1) return a.per[2] || (s >= 0 && s < nz);
-    return (a.per[0] || (ux >= 0 && ux < nx)) && (a.per[1] || (uy >= 0 && uy < ny)) &&
-           (a.per[2] || (s >= 0 && s < nz));
+  auto inside = [&](int ux, int uy, int s, auto mc) {
+    constexpr int M = decltype(mc)::value;
+    bool in = true;
+    if constexpr (tb::ring(M)) in = (a.per[0] || (ux >= 0 && ux < nx)) && (a.per[1] || (uy >= 0 && uy < ny));
+    if constexpr (tb::zfaces(M)) in = in && (a.per[2] || (s >= 0 && s < nz));
+    return in;
   };
   constexpr bool kPrefetch = sizeof(R) == 4 && (NT <= 512 || EPT1 == 1);
   R nxt[EPT1][19];
-  auto pull_plane = [&](int s) {
+  auto pull_plane = [&](int s, auto mc) {
+    constexpr int M = decltype(mc)::value;
     const int zs = tb::wrap(s, nz);
     const int zm = tb::wrap(zs - 1, nz), zp = tb::wrap(zs + 1, nz);
 #pragma unroll
     for (int r = 0; r < EPT1; ++r) {
       const int e = tid + r * NT;
-      if (e < N1 && inside(x0 - 2 + e % E1X, y0 - 2 + e / E1X, s)) {
+      if (e < N1 && inside(x0 - 2 + e % E1X, y0 - 2 + e / E1X, s, mc)) {
         const int ex = e % E1X, ey = e / E1X;
         const int gx = tb::wrap(x0 - 2 + ex, nx), gy = tb::wrap(y0 - 2 + ey, ny);
         const int xm = tb::wrap(gx - 1, nx), xp = tb::wrap(gx + 1, nx);
@@ -521,51 +561,52 @@ KMI_DEV void march3(const StepArgs& a, int zlen, int tx, int ty, int zc, typenam
         const unsigned bx[3] = {unsigned(xm) * ES, unsigned(gx) * ES, unsigned(xp) * ES};
         const int yy[3] = {ym, gy, yp}, zz[3] = {zm, zs, zp};
         tb::Nbr nb{};
-        if constexpr (BND) nb = tb::nbr<BND>(a, gx, gy, zs);
+        if constexpr (M != 0) nb = tb::nbr<M>(a, gx, gy, zs);
         const unsigned own = (unsigned(gx) + unsigned(nx) * unsigned(gy + ny * zs)) * ES;
         sfor<19>([&](auto qc) {
           constexpr int q = decltype(qc)::value;
           constexpr int cx = Lat<19>::cx[q], cy = Lat<19>::cy[q], cz = Lat<19>::cz[q];
-          bool ok = true;
-          if constexpr (BND) ok = tb::src_ok<q>(nb);
-          if (ok) {
-            const unsigned row = unsigned(nx) * unsigned(yy[1 - cy] + ny * zz[1 - cz]) * ES;
-            nxt[r][q] = Pops<ST>::ld(&tb::at(fi + q * P, row + bx[1 - cx]));
-          } else if constexpr (BND) {
-            R v = Pops<ST>::ld(&tb::at(fi + Lat<19>::opp[q] * P, own));
-            if constexpr (q != 0)
-              if (a.any_moving) v = tb::ladd<q, BND>(v, a, nb);
-            nxt[r][q] = v;
+          const unsigned row = unsigned(nx) * unsigned(yy[1 - cy] + ny * zz[1 - cz]) * ES;
+          const E* plane = fi + q * P;
+          unsigned off = row + bx[1 - cx];
+          if constexpr (M != 0 && q != 0) {
+            const bool ok = tb::src_ok<q>(nb);
+            plane = ok ? plane : fi + Lat<19>::opp[q] * P;
+            off = ok ? off : own;
           }
+          nxt[r][q] = Pops<ST>::ld(&tb::at(plane, off));
         });
       }
     }
   };
-  if constexpr (kPrefetch) pull_plane(z0 - 2);
+  if constexpr (kPrefetch) pull_plane(z0 - 2, std::integral_constant<int, BND>{});
   // two-barrier schedule: the c_z = +1 values of the previous plane, held one plane longer
   R k1q[TWO ? EPT1 : 1][5] = {}, k2q[TWO ? EPT2 : 1][5] = {};
 
-  for (int s = z0 - 2; s <= z1 + 1; ++s) {
+  // One plane of the march; M: the mode of its cells (BND, or its form off the z faces).
+  auto iterate = [&](int s, auto mc) {
+    constexpr int M = decltype(mc)::value;
     const int u = s + 4;  // non-negative plane counter for the ring slots
     R* const C1w = C1 + (BND ? (u & 1) : 0) * 5 * N1;        // c_z = −1, level 1, plane s
     R* const C2w = C2 + (BND ? ((u - 1) & 1) : 0) * 5 * N2;  // c_z = −1, level 2, plane s−1
     // ---- P1: t+1 on plane s, level-1 tile ----
-    if constexpr (!kPrefetch) pull_plane(s);
+    if constexpr (!kPrefetch) pull_plane(s, mc);
     R cur[EPT1][19];
 #pragma unroll
     for (int r = 0; r < EPT1; ++r)
 #pragma unroll
       for (int q = 0; q < 19; ++q) cur[r][q] = nxt[r][q];
     if constexpr (kPrefetch)
-      if (s <= z1) pull_plane(s + 1);
+      if (s <= z1) pull_plane(s + 1, mc);
     R k1z[EPT1][9], k1p[EPT1][5];
 #pragma unroll
     for (int r = 0; r < EPT1; ++r) {
       const int e = tid + r * NT;
-      if (e < N1 && inside(x0 - 2 + e % E1X, y0 - 2 + e / E1X, s)) {
+      if (e < N1 && inside(x0 - 2 + e % E1X, y0 - 2 + e / E1X, s, mc)) {
         R fn[19];
-        update19<ST, COLL, BND>(cur[r], fn, a, tb::wrap(x0 - 2 + e % E1X, nx), tb::wrap(y0 - 2 + e / E1X, ny),
-                                tb::wrap(s, nz));
+        const int gx = tb::wrap(x0 - 2 + e % E1X, nx), gy = tb::wrap(y0 - 2 + e / E1X, ny), gz = tb::wrap(s, nz);
+        if constexpr (M != 0) tb::ladd_all<M>(cur[r], a, tb::nbr<M>(a, gx, gy, gz));
+        update19<ST, COLL, M>(cur[r], fn, a, gx, gy, gz);
         sfor<19>([&](auto qc) {
           constexpr int q = decltype(qc)::value;
           constexpr int cz = Lat<19>::cz[q];
@@ -587,14 +628,14 @@ KMI_DEV void march3(const StepArgs& a, int zlen, int tx, int ty, int zc, typenam
 #pragma unroll
       for (int r = 0; r < EPT2; ++r) {
         const int e = tid + r * NT;
-        if (e < N2 && inside(x0 - 1 + e % E2X, y0 - 1 + e / E2X, s - 1)) {
+        if (e < N2 && inside(x0 - 1 + e % E2X, y0 - 1 + e / E2X, s - 1, mc)) {
           const int ex = e % E2X, ey = e / E2X;
           const int gx = tb::wrap(x0 - 1 + ex, nx), gy = tb::wrap(y0 - 1 + ey, ny), gz = tb::wrap(s - 1, nz);
           tb::Nbr nb{};
-          if constexpr (BND) nb = tb::nbr<BND>(a, gx, gy, gz);
+          if constexpr (M != 0) nb = tb::nbr<M>(a, gx, gy, gz);
           R fp[19], fn[19];
-          pull_lds<BND>(fp, A1, B1r, C1w, B1o, C1o, N1, E1X, ex + 1, ey + 1, a, nb);
-          update19<ST, COLL, BND>(fp, fn, a, gx, gy, gz);
+          pull_lds<M>(fp, A1, B1r, C1w, B1o, C1o, N1, E1X, ex + 1, ey + 1, a, nb);
+          update19<ST, COLL, M>(fp, fn, a, gx, gy, gz);
           sfor<19>([&](auto qc) {
             constexpr int q = decltype(qc)::value;
             constexpr int cz = Lat<19>::cz[q];
@@ -620,10 +661,10 @@ KMI_DEV void march3(const StepArgs& a, int zlen, int tx, int ty, int zc, typenam
       const R* const C2o = C2 + (BND ? ((u - 2) & 1) : 0) * 5 * N2;  // c_z = −1 of plane s−2 (own)
       const int ix = tid % TX, iy = tid / TX;
       tb::Nbr nb{};
-      if constexpr (BND) nb = tb::nbr<BND>(a, x0 + ix, y0 + iy, s - 2);
+      if constexpr (M != 0) nb = tb::nbr<M>(a, x0 + ix, y0 + iy, s - 2);
       R fp[19], fn[19];
-      pull_lds<BND>(fp, A2r, B2r, C2w, B2o, C2o, N2, E2X, ix + 1, iy + 1, a, nb);
-      update19<ST, COLL, BND>(fp, fn, a, x0 + ix, y0 + iy, s - 2);
+      pull_lds<M>(fp, A2r, B2r, C2w, B2o, C2o, N2, E2X, ix + 1, iy + 1, a, nb);
+      update19<ST, COLL, M>(fp, fn, a, x0 + ix, y0 + iy, s - 2);
       const unsigned cell = (unsigned(x0 + ix) + unsigned(nx) * unsigned(y0 + iy + ny * (s - 2))) * ES;
       sfor<19>([&](auto qc) {
         constexpr int q = decltype(qc)::value;
@@ -677,7 +718,7 @@ KMI_DEV void march3(const StepArgs& a, int zlen, int tx, int ty, int zc, typenam
 #pragma unroll
         for (int r = 0; r < EPT1; ++r) {
           const int e = tid + r * NT;
-          if (e < N1 && inside(x0 - 2 + e % E1X, y0 - 2 + e / E1X, s)) {
+          if (e < N1 && inside(x0 - 2 + e % E1X, y0 - 2 + e / E1X, s, mc)) {
 #pragma unroll
             for (int n = 0; n < 9; ++n) A1[n * N1 + e] = k1z[r][n];
 #pragma unroll
@@ -692,7 +733,7 @@ KMI_DEV void march3(const StepArgs& a, int zlen, int tx, int ty, int zc, typenam
 #pragma unroll
         for (int r = 0; r < EPT2; ++r) {
           const int e = tid + r * NT;
-          if (e < N2 && inside(x0 - 1 + e % E2X, y0 - 1 + e / E2X, s - 1)) {
+          if (e < N2 && inside(x0 - 1 + e % E2X, y0 - 1 + e / E2X, s - 1, mc)) {
 #pragma unroll
             for (int n = 0; n < 9; ++n) A2[n * N2 + e] = k2z[r][n];
 #pragma unroll
@@ -701,7 +742,8 @@ KMI_DEV void march3(const StepArgs& a, int zlen, int tx, int ty, int zc, typenam
         }
       }
     }
-  }
+  };
+  march_planes<BND, 3>(a, z0 - 2, z1 + 1, nz, iterate);
 }
 
 // Grid and walled tiles as for k_step2_d3q19.
