@@ -242,6 +242,9 @@ struct StepArgs {
   // Walled multi-step launches: work-group b marches tile tile_order[b] (-1: padding);
   // nullptr: the XCD-banded order of the periodic launches.
   const int* tile_order;
+  // Single-step launches in whole rows: rows of a plane are dealt out in 2^xcd_shift bands,
+  // one per XCD (the grid's y extent is a multiple of 8).
+  int xcd_shift;
   FaceArgs face[6];
 };
 
