@@ -99,12 +99,15 @@ int kmi_ctx_create(int device, kmi_ctx** out) {
   if (!c) return fail(nullptr, KMI_ERR_NOMEM, "kmi_ctx_create: out of host memory");
   c->device = device;
   if ((e = hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking)) != hipSuccess ||
-      (e = hipMalloc(&c->partials, 2048 * 3 * 2 * sizeof(double))) != hipSuccess ||
-      (e = hipMalloc(&c->out, 8 * sizeof(double))) != hipSuccess ||
-      (e = resolve_noalloc_workspace(device)) != hipSuccess) {
+      (e = hipMalloc(&c->partials, (kRedPartials + 1) * sizeof(double))) != hipSuccess ||
+      (e = hipMemset(c->partials, 0, (kRedPartials + 1) * sizeof(double))) != hipSuccess ||
+      (e = hipDeviceSynchronize()) != hipSuccess ||
+      (e = hipHostMalloc(reinterpret_cast<void**>(&c->out), 8 * sizeof(double), hipHostMallocDefault)) != hipSuccess ||
+      (e = resolve_noalloc_workspace(device)) != hipSuccess ||
+      (e = (c->copier = host_copier_create()) ? hipSuccess : hipErrorOutOfMemory) != hipSuccess) {
     if (c->stream) (void)hipStreamDestroy(c->stream);
     if (c->partials) (void)hipFree(c->partials);
-    if (c->out) (void)hipFree(c->out);
+    if (c->out) (void)hipHostFree(c->out);
     delete c;
     return hip_fail(nullptr, e, "kmi_ctx_create");
   }
@@ -117,8 +120,9 @@ int kmi_ctx_destroy(kmi_ctx* ctx) {
   if (!ctx) return KMI_OK;
   (void)hipSetDevice(ctx->device);
   (void)hipStreamSynchronize(ctx->stream);
+  host_copier_destroy(ctx->copier);
   (void)hipFree(ctx->partials);
-  (void)hipFree(ctx->out);
+  (void)hipHostFree(ctx->out);
   (void)hipStreamDestroy(ctx->stream);
   delete ctx;
   return KMI_OK;
@@ -890,8 +894,9 @@ int kmi_upload(kmi_lattice* L, int32_t field, const void* host, int32_t host_dty
   KMI_HIP(c, hipSetDevice(c->device));
   const size_t n = size_t(L->ncells) * L->Q;
   if (host_dtype == KMI_HOST_STORAGE) {  // storage elements verbatim (planes are unpadded)
+    const HostSeg seg{const_cast<void*>(host), buf[L->cur], n * storage_bytes(st)};
+    KMI_HIP(c, copy_to_device(c, &seg, 1));
     KMI_HIP(c, hipStreamSynchronize(c->stream));
-    KMI_HIP(c, hipMemcpy(buf[L->cur], host, n * storage_bytes(st), hipMemcpyHostToDevice));
     if (field == KMI_FIELD_F) L->steps = 0;
     return KMI_OK;
   }
@@ -905,7 +910,8 @@ int kmi_upload(kmi_lattice* L, int32_t field, const void* host, int32_t host_dty
   }
   double* stage = nullptr;
   KMI_HIP(c, stage_reserve(L, n * sizeof(double), &stage));
-  hipError_t e = hipMemcpyAsync(stage, src, n * sizeof(double), hipMemcpyHostToDevice, c->stream);
+  const HostSeg seg{const_cast<double*>(src), stage, n * sizeof(double)};
+  hipError_t e = copy_to_device(c, &seg, 1);
   if (e == hipSuccess)
     e = launch_to_storage(L->Q, st, stage, buf[L->cur], L->ncells, L->plane, shift, c->stream);
   if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
@@ -927,8 +933,8 @@ int kmi_download(kmi_lattice* L, int32_t field, void* host, int32_t host_dtype) 
   KMI_HIP(c, hipSetDevice(c->device));
   const size_t n = size_t(L->ncells) * L->Q;
   if (host_dtype == KMI_HOST_STORAGE) {
-    KMI_HIP(c, hipStreamSynchronize(c->stream));
-    KMI_HIP(c, hipMemcpy(host, buf[L->cur], n * storage_bytes(st), hipMemcpyDeviceToHost));
+    const HostSeg seg{host, buf[L->cur], n * storage_bytes(st)};
+    KMI_HIP(c, copy_to_host(c, &seg, 1));
     return KMI_OK;
   }
   double* stage = nullptr;
@@ -941,9 +947,8 @@ int kmi_download(kmi_lattice* L, int32_t field, void* host, int32_t host_dtype) 
   }
   hipError_t e = launch_from_storage(L->Q, st, buf[L->cur], stage, L->ncells, L->plane, shift,
                                      c->stream);
-  if (e == hipSuccess)
-    e = hipMemcpyAsync(dst, stage, n * sizeof(double), hipMemcpyDeviceToHost, c->stream);
-  if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
+  const HostSeg seg{dst, stage, n * sizeof(double)};
+  if (e == hipSuccess) e = copy_to_host(c, &seg, 1);
   if (e != hipSuccess) return hip_fail(c, e, "kmi_download");
   if (host_dtype == KMI_HOST_F32) {
     float* h = static_cast<float*>(host);
@@ -963,14 +968,14 @@ static int stage_fields(kmi_lattice* L, const double* const* host, int count, do
   for (int k = 0; k < count; ++k) dev[k] = nullptr;
   if (used == 0) return KMI_OK;
   KMI_HIP(c, stage_reserve(L, size_t(used) * L->ncells * sizeof(double), &block));
+  HostSeg seg[5];
   int slot = 0;
   for (int k = 0; k < count; ++k) {
     if (!host[k]) continue;
-    dev[k] = block + size_t(slot++) * L->ncells;
-    hipError_t e = hipMemcpyAsync(dev[k], host[k], size_t(L->ncells) * sizeof(double),
-                                  hipMemcpyHostToDevice, c->stream);
-    if (e != hipSuccess) return hip_fail(c, e, "staging host field");
+    dev[k] = block + size_t(slot) * L->ncells;
+    seg[slot++] = HostSeg{const_cast<double*>(host[k]), dev[k], size_t(L->ncells) * sizeof(double)};
   }
+  if (hipError_t e = copy_to_device(c, seg, slot); e != hipSuccess) return hip_fail(c, e, "staging host field");
   return KMI_OK;
 }
 
@@ -1049,8 +1054,8 @@ static int reduce_cells(kmi_lattice* L, int kind, double* out3) {
                                      c->partials, c->out, c->stream);
   if (e != hipSuccess) return hip_fail(c, e, "reduction kernel");
   if (kind == 101) return KMI_OK;
-  KMI_HIP(c, hipMemcpyAsync(out3, c->out, 3 * sizeof(double), hipMemcpyDeviceToHost, c->stream));
   KMI_HIP(c, hipStreamSynchronize(c->stream));
+  std::copy_n(c->out, 3, out3);
   return KMI_OK;
 }
 
@@ -1105,11 +1110,11 @@ int kmi_moments(kmi_lattice* L, double* rho, double* ux, double* uy, double* uz,
                                 L->desc.thermal ? L->g[L->cur] : nullptr, dev[0], dev[1], dev[2],
                                 dev[3], dev[4], L->ncells, L->plane, L->desc.T_ref, mom_force(L),
                                 c->stream);
-  for (int k = 0; k < 5 && e == hipSuccess; ++k)
-    if (host[k])
-      e = hipMemcpyAsync(host[k], dev[k], size_t(L->ncells) * sizeof(double),
-                         hipMemcpyDeviceToHost, c->stream);
-  if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
+  HostSeg seg[5];
+  slot = 0;
+  for (int k = 0; k < 5; ++k)
+    if (host[k]) seg[slot++] = HostSeg{host[k], dev[k], size_t(L->ncells) * sizeof(double)};
+  if (e == hipSuccess) e = copy_to_host(c, seg, slot);
   if (e != hipSuccess) return hip_fail(c, e, "kmi_moments");
   return KMI_OK;
 }
@@ -1171,8 +1176,8 @@ int kmi_reduce(kmi_lattice* L, int32_t kind, int32_t arg, double* out) {
                                     int(n[2]), L->plane, d.T_ref, arg, Th, dT, lo1, hi1, lo2, hi2,
                                     c->partials, c->out, c->stream);
       if (e != hipSuccess) return hip_fail(c, e, "Nusselt kernel");
-      KMI_HIP(c, hipMemcpyAsync(r, c->out, sizeof(double), hipMemcpyDeviceToHost, c->stream));
       KMI_HIP(c, hipStreamSynchronize(c->stream));
+      r[0] = c->out[0];
       out[0] = r[0] / double(int64_t(hi1 - lo1) * (hi2 - lo2));
       return KMI_OK;
     }
@@ -1185,8 +1190,8 @@ int kmi_reduce(kmi_lattice* L, int32_t kind, int32_t arg, double* out) {
                                    L->args.nz, L->plane, kind == KMI_RED_DRAG_MEA, c->partials,
                                    c->out, c->stream);
         if (e != hipSuccess) return hip_fail(c, e, "drag kernel");
-        KMI_HIP(c, hipMemcpyAsync(r, c->out, 3 * sizeof(double), hipMemcpyDeviceToHost, c->stream));
         KMI_HIP(c, hipStreamSynchronize(c->stream));
+        std::copy_n(c->out, 3, r);
       }
       out[0] = r[0];
       out[1] = r[1];

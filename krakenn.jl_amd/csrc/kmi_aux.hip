@@ -2,15 +2,19 @@
 //
 // Reductions are deterministic and compensated at every level: each thread accumulates its
 // cells in FP64 as a Neumaier pair (sum, error), a wave64 butterfly (__shfl_xor) and an LDS
-// pass across waves merge the pairs, each work-group writes its pair, and one 256-thread
-// work-group folds the group pairs (strided per thread, then a fixed LDS tree).  No atomics,
-// so repeated calls return identical bits.
-#include "kmi_common.h"
+// pass across waves merge the pairs, each work-group writes its pair, and one work-group (the
+// one that finishes last, or a second launch) folds the group pairs (strided per thread, then a fixed LDS tree): the order of
+// the sums does not depend on which group that is, so repeated calls return identical bits.
+// The result goes to host memory, so a call needs no copy.  Up to kFusedGroups groups a call is
+// one launch; beyond, the fence of every group (it writes the XCD's L2 back) costs more than a
+// second launch (mass of 2048² F64: 165 µs fused, 82 as two launches).
+#include "kmi_internal.h"
 
 namespace kmi {
 
 constexpr int kRedBlock = 256;
 constexpr int kRedMaxVals = 4;
+constexpr int kFusedGroups = 16;
 
 // --- conversion host layout (double, [cell, q]) <-> storage ------------------------------
 // shift_q: w_q for f, w_q T_ref for g (shifted storage only).
@@ -211,13 +215,84 @@ KMI_DEV void block_reduce(double (&v)[NV], double (&c)[NV], bool is_max, double*
   }
 }
 
+// Combine the `nb` group pairs of `nv` values: thread t folds groups t, t + 256, … in order,
+// then a fixed LDS tree merges the 256 thread pairs.  One work-group of 256 threads.
+KMI_DEV void finalize(const double* partials, int nb, int nv, bool is_max, double* out) {
+  __shared__ double ls[kRedBlock], lc[kRedBlock];
+  const int t = threadIdx.x;
+  for (int n = 0; n < nv; ++n) {
+    double s = is_max ? -HUGE_VAL : 0.0, c = 0.0;
+    for (int b = t; b < nb; b += kRedBlock) {
+      const double x = partials[2 * (b * nv + n)], e = partials[2 * (b * nv + n) + 1];
+      if (is_max) s = fmax(s, x);
+      else nsum_merge(s, c, x, e);
+    }
+    ls[t] = s;
+    lc[t] = c;
+    __syncthreads();
+    int w = kRedBlock / 2;
+    while (w >= nb) w >>= 1;  // merging the empty pairs beyond nb changes nothing
+    for (; w > 0; w >>= 1) {
+      if (t < w) {
+        if (is_max) {
+          ls[t] = fmax(ls[t], ls[t + w]);
+        } else {
+          double a = ls[t], ac = lc[t];
+          nsum_merge(a, ac, ls[t + w], lc[t + w]);
+          ls[t] = a;
+          lc[t] = ac;
+        }
+      }
+      __syncthreads();
+    }
+    if (t == 0) out[n] = is_max ? ls[0] : ls[0] + lc[0];
+    __syncthreads();
+  }
+}
+
+// Groups done so far, behind the partials; zero between launches.
+KMI_DEV unsigned* done_counter(double* partials) {
+  return reinterpret_cast<unsigned*>(partials + kRedPartials);
+}
+
+// The group's pairs of NV values; in a launch of up to kFusedGroups groups also the final sums,
+// from the group that is last to write its own.  The fences order the pairs before the count
+// and the count before the reads of the other groups' pairs, across the XCDs' caches.
+template <int NV>
+KMI_DEV void reduce_to(double (&v)[NV], double (&c)[NV], bool is_max, double* partials, double* out) {
+  __shared__ bool last;
+  block_reduce<NV>(v, c, is_max, partials);
+  if (gridDim.x > kFusedGroups) return;
+  if (threadIdx.x == 0) {
+    __threadfence();
+    last = atomicAdd(done_counter(partials), 1u) == gridDim.x - 1;
+  }
+  __syncthreads();
+  if (!last) return;
+  __threadfence();
+  if (threadIdx.x == 0) *done_counter(partials) = 0u;
+  finalize(partials, int(gridDim.x), NV, is_max, out);
+}
+
+__global__ void __launch_bounds__(kRedBlock) k_finalize(const double* __restrict__ partials, int nb, int nv,
+                                                        int is_max, double* __restrict__ out) {
+  finalize(partials, nb, nv, is_max != 0, out);
+}
+
+static hipError_t finish_reduction(const double* partials, int nb, int nv, bool is_max, double* out, hipStream_t s) {
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess || nb <= kFusedGroups) return e;
+  hipLaunchKernelGGL(k_finalize, dim3(1), dim3(kRedBlock), 0, s, partials, nb, nv, is_max ? 1 : 0, out);
+  return hipGetLastError();
+}
+
 // kind: 0 mass, 1 momentum, 2 kinetic energy, 3 thermal, 5 max speed,
 //       100 residual (Σ fluid |u − u_prev|², Σ fluid |u|²), 101 snapshot u → u_prev.
 template <int Q, int ST>
 __global__ void __launch_bounds__(kRedBlock)
     k_reduce_cells(const void* f, const void* g, const uint8_t* mask, double* uprev,
                    long long ncells, long long plane, double T0, MomForce F, int kind,
-                   double* partials) {
+                   double* partials, double* out) {
   double acc[3] = {0.0, 0.0, 0.0}, err[3] = {0.0, 0.0, 0.0};
   const bool is_max = kind == KMI_RED_MAX_SPEED;
   for (long long c = (long long)blockIdx.x * blockDim.x + threadIdx.x; c < ncells;
@@ -250,7 +325,7 @@ __global__ void __launch_bounds__(kRedBlock)
     }
   }
   if (kind == 101) return;
-  block_reduce<3>(acc, err, is_max, partials);
+  reduce_to<3>(acc, err, is_max, partials, out);
 }
 
 // Hot-wall Nusselt number per wall node (thermal.jl:225-234, 525-533):
@@ -260,7 +335,7 @@ __global__ void __launch_bounds__(kRedBlock)
 template <int Q, int ST>
 __global__ void __launch_bounds__(kRedBlock)
     k_nusselt(const void* g_, int nx, int ny, int nz, long long plane, double T0, int face,
-              double Th, double dT, int lo1, int hi1, int lo2, int hi2, double* partials) {
+              double Th, double dT, int lo1, int hi1, int lo2, int hi2, double* partials, double* out) {
   using S = Store<ST>;
   using E = typename S::elem;
   const E* g = static_cast<const E*>(g_);
@@ -293,7 +368,7 @@ __global__ void __launch_bounds__(kRedBlock)
     }
     nsum_add(acc[0], err[0], -H * (-8 * Th + 9 * T1 - T2) / 3.0 / dT);
   }
-  block_reduce<1>(acc, err, false, partials);
+  reduce_to<1>(acc, err, false, partials, out);
 }
 
 // Force on the cut-link walls, accumulated in FP64 over the link list.
@@ -308,7 +383,7 @@ __global__ void __launch_bounds__(kRedBlock)
     k_drag(const void* f_, long long nlinks, const int* __restrict__ cell,
            const int* __restrict__ qv, const double* __restrict__ qwv,
            const double* __restrict__ uwv, int nx, int ny, int nz, long long plane, int mea,
-           double* partials) {
+           double* partials, double* out) {
   using S = Store<ST>;
   using E = typename S::elem;
   const E* f = static_cast<const E*>(f_);
@@ -362,41 +437,7 @@ __global__ void __launch_bounds__(kRedBlock)
     nsum_add(acc[1], err[1], double(cy) * F);
     nsum_add(acc[2], err[2], double(cz) * F);
   }
-  block_reduce<3>(acc, err, false, partials);
-}
-
-// Combine the `nb` group pairs of `nv` values: thread t folds groups t, t + 256, … in order,
-// then a fixed LDS tree merges the 256 thread pairs.  One work-group of 256 threads.
-__global__ void __launch_bounds__(256) k_finalize(const double* __restrict__ partials, int nb, int nv,
-                                                  int is_max, double* __restrict__ out) {
-  __shared__ double ls[256], lc[256];
-  const int t = threadIdx.x;
-  for (int n = 0; n < nv; ++n) {
-    double s = is_max ? -HUGE_VAL : 0.0, c = 0.0;
-    for (int b = t; b < nb; b += 256) {
-      const double x = partials[2 * (b * nv + n)], e = partials[2 * (b * nv + n) + 1];
-      if (is_max) s = fmax(s, x);
-      else nsum_merge(s, c, x, e);
-    }
-    ls[t] = s;
-    lc[t] = c;
-    __syncthreads();
-    for (int w = 128; w > 0; w >>= 1) {
-      if (t < w) {
-        if (is_max) {
-          ls[t] = fmax(ls[t], ls[t + w]);
-        } else {
-          double a = ls[t], ac = lc[t];
-          nsum_merge(a, ac, ls[t + w], lc[t + w]);
-          ls[t] = a;
-          lc[t] = ac;
-        }
-      }
-      __syncthreads();
-    }
-    if (t == 0) out[n] = is_max ? ls[0] : ls[0] + lc[0];
-    __syncthreads();
-  }
+  reduce_to<3>(acc, err, false, partials, out);
 }
 
 // Plain device copy (float4 loads, non-temporal float4 stores): the practical 1:1
@@ -467,7 +508,7 @@ hipError_t launch_moments(int Q, int st, const void* f, const void* g, double* r
 // Number of partial slots a reduction launch needs (3 values per group).
 int reduce_groups(long long ncells) {
   long long g = (ncells + kRedBlock - 1) / kRedBlock;
-  return int(g < 2048 ? (g < 1 ? 1 : g) : 2048);
+  return int(g < kRedGroups ? (g < 1 ? 1 : g) : kRedGroups);
 }
 
 hipError_t launch_reduce_cells(int Q, int st, const void* f, const void* g, const uint8_t* mask,
@@ -475,37 +516,28 @@ hipError_t launch_reduce_cells(int Q, int st, const void* f, const void* g, cons
                                const MomForce& F, int kind, double* partials, double* out,
                                hipStream_t s) {
   const int nb = reduce_groups(ncells);
-  if (Q == 9) { KMI_ST_SWITCH(st, hipLaunchKernelGGL((k_reduce_cells<9, ST>), dim3(nb), dim3(kRedBlock), 0, s, f, g, mask, uprev, ncells, plane, T0, F, kind, partials)); }
-  else { KMI_ST_SWITCH(st, hipLaunchKernelGGL((k_reduce_cells<19, ST>), dim3(nb), dim3(kRedBlock), 0, s, f, g, mask, uprev, ncells, plane, T0, F, kind, partials)); }
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess || kind == 101) return e;
-  hipLaunchKernelGGL(k_finalize, dim3(1), dim3(256), 0, s, partials, nb, 3,
-                     kind == KMI_RED_MAX_SPEED ? 1 : 0, out);
-  return hipGetLastError();
+  if (Q == 9) { KMI_ST_SWITCH(st, hipLaunchKernelGGL((k_reduce_cells<9, ST>), dim3(nb), dim3(kRedBlock), 0, s, f, g, mask, uprev, ncells, plane, T0, F, kind, partials, out)); }
+  else { KMI_ST_SWITCH(st, hipLaunchKernelGGL((k_reduce_cells<19, ST>), dim3(nb), dim3(kRedBlock), 0, s, f, g, mask, uprev, ncells, plane, T0, F, kind, partials, out)); }
+  if (kind == 101) return hipGetLastError();
+  return finish_reduction(partials, nb, 3, kind == KMI_RED_MAX_SPEED, out, s);
 }
 
 hipError_t launch_drag(int Q, int st, const void* f, long long nlinks, const int* cell,
                        const int* q, const double* qw, const double* uw, int nx, int ny, int nz,
                        long long plane, int mea, double* partials, double* out, hipStream_t s) {
   const int nb = reduce_groups(nlinks);
-  if (Q == 9) { KMI_ST_SWITCH(st, hipLaunchKernelGGL((k_drag<9, ST>), dim3(nb), dim3(kRedBlock), 0, s, f, nlinks, cell, q, qw, uw, nx, ny, nz, plane, mea, partials)); }
-  else { KMI_ST_SWITCH(st, hipLaunchKernelGGL((k_drag<19, ST>), dim3(nb), dim3(kRedBlock), 0, s, f, nlinks, cell, q, qw, uw, nx, ny, nz, plane, mea, partials)); }
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(k_finalize, dim3(1), dim3(256), 0, s, partials, nb, 3, 0, out);
-  return hipGetLastError();
+  if (Q == 9) { KMI_ST_SWITCH(st, hipLaunchKernelGGL((k_drag<9, ST>), dim3(nb), dim3(kRedBlock), 0, s, f, nlinks, cell, q, qw, uw, nx, ny, nz, plane, mea, partials, out)); }
+  else { KMI_ST_SWITCH(st, hipLaunchKernelGGL((k_drag<19, ST>), dim3(nb), dim3(kRedBlock), 0, s, f, nlinks, cell, q, qw, uw, nx, ny, nz, plane, mea, partials, out)); }
+  return finish_reduction(partials, nb, 3, false, out, s);
 }
 
 hipError_t launch_nusselt(int Q, int st, const void* g, int nx, int ny, int nz, long long plane,
                           double T0, int face, double Th, double dT, int lo1, int hi1, int lo2,
                           int hi2, double* partials, double* out, hipStream_t s) {
   const int nb = reduce_groups((long long)(hi1 - lo1) * (hi2 - lo2));
-  if (Q == 9) { KMI_ST_SWITCH(thermal_storage(st), hipLaunchKernelGGL((k_nusselt<9, ST>), dim3(nb), dim3(kRedBlock), 0, s, g, nx, ny, nz, plane, T0, face, Th, dT, lo1, hi1, lo2, hi2, partials)); }
-  else { KMI_ST_SWITCH(thermal_storage(st), hipLaunchKernelGGL((k_nusselt<19, ST>), dim3(nb), dim3(kRedBlock), 0, s, g, nx, ny, nz, plane, T0, face, Th, dT, lo1, hi1, lo2, hi2, partials)); }
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(k_finalize, dim3(1), dim3(256), 0, s, partials, nb, 1, 0, out);
-  return hipGetLastError();
+  if (Q == 9) { KMI_ST_SWITCH(thermal_storage(st), hipLaunchKernelGGL((k_nusselt<9, ST>), dim3(nb), dim3(kRedBlock), 0, s, g, nx, ny, nz, plane, T0, face, Th, dT, lo1, hi1, lo2, hi2, partials, out)); }
+  else { KMI_ST_SWITCH(thermal_storage(st), hipLaunchKernelGGL((k_nusselt<19, ST>), dim3(nb), dim3(kRedBlock), 0, s, g, nx, ny, nz, plane, T0, face, Th, dT, lo1, hi1, lo2, hi2, partials, out)); }
+  return finish_reduction(partials, nb, 1, false, out, s);
 }
 
 }  // namespace kmi

@@ -496,6 +496,8 @@ struct kmi_batch {
   double* partials = nullptr;
   size_t partials_cap = 0;
   double* resid_d = nullptr;  // 3 per cavity
+  double* stage = nullptr;    // device staging of host transfers (grown on demand, kept)
+  size_t stage_bytes = 0;
   std::vector<int> status;
   std::vector<int64_t> steps;
   std::vector<double> resid;
@@ -802,7 +804,7 @@ int kmi_batch_destroy(kmi_batch* B) {
   (void)hipStreamSynchronize(B->ctx->stream);
   batch_drop_graphs(B);
   void* ptrs[] = {B->f[0], B->f[1], B->cav_d, B->slots_d, B->cav_slots_d, B->cav_range_d,
-                  B->pieces_d, B->active_d, B->uprev, B->partials, B->resid_d};
+                  B->pieces_d, B->stage, B->active_d, B->uprev, B->partials, B->resid_d};
   for (void* p : ptrs)
     if (p) (void)hipFree(p);
   for (auto ev : B->ev)
@@ -820,6 +822,17 @@ static hipError_t batch_mirror_if_retired(kmi_batch* B, int32_t c, hipStream_t s
   return hipMemcpyAsync(static_cast<char*>(B->f[B->cur ^ 1]) + off,
                         static_cast<const char*>(B->f[B->cur]) + off, bytes,
                         hipMemcpyDeviceToDevice, s);
+}
+
+static hipError_t batch_stage(kmi_batch* B, size_t bytes) {
+  if (B->stage_bytes >= bytes) return hipSuccess;
+  hipError_t e = hipStreamSynchronize(B->ctx->stream);
+  if (e != hipSuccess) return e;
+  if (B->stage) (void)hipFree(B->stage);
+  B->stage = nullptr;
+  B->stage_bytes = 0;
+  if ((e = hipMalloc(&B->stage, bytes)) == hipSuccess) B->stage_bytes = bytes;
+  return e;
 }
 
 static int batch_check_cav(kmi_batch* B, int32_t c) {
@@ -841,14 +854,14 @@ int kmi_batch_upload(kmi_batch* B, int32_t c, const void* host, int32_t dt) {
     for (long long i = 0; i < 9 * nc; ++i) tmp[i] = static_cast<const float*>(host)[i];
     src = tmp.data();
   }
-  double* stage = nullptr;
-  KMI_HIP(x, hipMalloc(&stage, size_t(9 * nc) * sizeof(double)));
-  hipError_t e = hipMemcpyAsync(stage, src, size_t(9 * nc) * sizeof(double), hipMemcpyHostToDevice, x->stream);
+  KMI_HIP(x, batch_stage(B, size_t(9 * nc) * sizeof(double)));
+  double* const stage = B->stage;
+  const HostSeg seg{const_cast<double*>(src), stage, size_t(9 * nc) * sizeof(double)};
+  hipError_t e = copy_to_device(x, &seg, 1);
   char* base = static_cast<char*>(B->f[B->cur]) + B->cav[c].foff * B->esize;
   if (e == hipSuccess) e = launch_to_storage(9, B->desc.storage, stage, base, nc, nc, 1.0, x->stream);
   if (e == hipSuccess) e = batch_mirror_if_retired(B, c, x->stream);
   if (e == hipSuccess) e = hipStreamSynchronize(x->stream);
-  (void)hipFree(stage);
   if (e != hipSuccess) return hip_fail(x, e, "kmi_batch_upload");
   return KMI_OK;
 }
@@ -859,8 +872,8 @@ int kmi_batch_download(kmi_batch* B, int32_t c, void* host, int32_t dt) {
   if (!host || (dt != KMI_HOST_F64 && dt != KMI_HOST_F32)) return fail(x, KMI_ERR_ARG, "kmi_batch_download: bad buffer");
   KMI_HIP(x, hipSetDevice(x->device));
   const long long nc = (long long)B->n[c] * B->n[c];
-  double* stage = nullptr;
-  KMI_HIP(x, hipMalloc(&stage, size_t(9 * nc) * sizeof(double)));
+  KMI_HIP(x, batch_stage(B, size_t(9 * nc) * sizeof(double)));
+  double* const stage = B->stage;
   std::vector<double> tmp;
   double* dst = static_cast<double*>(host);
   if (dt == KMI_HOST_F32) {
@@ -869,9 +882,8 @@ int kmi_batch_download(kmi_batch* B, int32_t c, void* host, int32_t dt) {
   }
   const char* base = static_cast<const char*>(B->f[B->cur]) + B->cav[c].foff * B->esize;
   hipError_t e = launch_from_storage(9, B->desc.storage, base, stage, nc, nc, 1.0, x->stream);
-  if (e == hipSuccess) e = hipMemcpyAsync(dst, stage, size_t(9 * nc) * sizeof(double), hipMemcpyDeviceToHost, x->stream);
-  if (e == hipSuccess) e = hipStreamSynchronize(x->stream);
-  (void)hipFree(stage);
+  const HostSeg seg{dst, stage, size_t(9 * nc) * sizeof(double)};
+  if (e == hipSuccess) e = copy_to_host(x, &seg, 1);
   if (e != hipSuccess) return hip_fail(x, e, "kmi_batch_download");
   if (dt == KMI_HOST_F32)
     for (long long i = 0; i < 9 * nc; ++i) static_cast<float*>(host)[i] = float(tmp[i]);
@@ -886,21 +898,22 @@ int kmi_batch_init_equilibrium(kmi_batch* B, int32_t c, const double* rho, const
   const long long nc = (long long)B->n[c] * B->n[c];
   const double* host[3] = {rho, ux, uy};
   double* dev[3] = {nullptr, nullptr, nullptr};
-  double* block = nullptr;
+  HostSeg seg[3];
   int used = 0;
   for (auto h : host) used += h != nullptr;
-  if (used) KMI_HIP(x, hipMalloc(&block, size_t(used) * nc * sizeof(double)));
+  if (used) KMI_HIP(x, batch_stage(B, size_t(used) * nc * sizeof(double)));
   hipError_t e = hipSuccess;
-  for (int k = 0, slot = 0; k < 3 && e == hipSuccess; ++k) {
+  used = 0;
+  for (int k = 0; k < 3; ++k) {
     if (!host[k]) continue;
-    dev[k] = block + size_t(slot++) * nc;
-    e = hipMemcpyAsync(dev[k], host[k], size_t(nc) * sizeof(double), hipMemcpyHostToDevice, x->stream);
+    dev[k] = B->stage + size_t(used) * nc;
+    seg[used++] = HostSeg{const_cast<double*>(host[k]), dev[k], size_t(nc) * sizeof(double)};
   }
+  if (used) e = copy_to_device(x, seg, used);
   char* base = static_cast<char*>(B->f[B->cur]) + B->cav[c].foff * B->esize;
   if (e == hipSuccess) e = launch_init_eq(9, B->desc.storage, base, dev[0], dev[1], dev[2], nullptr, nc, nc, x->stream);
   if (e == hipSuccess) e = batch_mirror_if_retired(B, c, x->stream);
   if (e == hipSuccess) e = hipStreamSynchronize(x->stream);
-  if (block) (void)hipFree(block);
   if (e != hipSuccess) return hip_fail(x, e, "kmi_batch_init_equilibrium");
   return KMI_OK;
 }
@@ -910,17 +923,18 @@ int kmi_batch_moments(kmi_batch* B, int32_t c, double* rho, double* ux, double* 
   kmi_ctx* x = B->ctx;
   KMI_HIP(x, hipSetDevice(x->device));
   const long long nc = (long long)B->n[c] * B->n[c];
-  double* block = nullptr;
-  KMI_HIP(x, hipMalloc(&block, size_t(3) * nc * sizeof(double)));
+  KMI_HIP(x, batch_stage(B, size_t(3) * nc * sizeof(double)));
+  double* const block = B->stage;
   const char* base = static_cast<const char*>(B->f[B->cur]) + B->cav[c].foff * B->esize;
   hipError_t e = launch_moments(9, B->desc.storage, base, nullptr, block, block + nc, block + 2 * nc,
                                 nullptr, nullptr, nc, nc, 0.0, MomForce{{0.0, 0.0, 0.0}, nullptr},
                                 x->stream);
   double* host[3] = {rho, ux, uy};
-  for (int k = 0; k < 3 && e == hipSuccess; ++k)
-    if (host[k]) e = hipMemcpyAsync(host[k], block + k * nc, size_t(nc) * sizeof(double), hipMemcpyDeviceToHost, x->stream);
-  if (e == hipSuccess) e = hipStreamSynchronize(x->stream);
-  (void)hipFree(block);
+  HostSeg seg[3];
+  int used = 0;
+  for (int k = 0; k < 3; ++k)
+    if (host[k]) seg[used++] = HostSeg{host[k], block + k * nc, size_t(nc) * sizeof(double)};
+  if (e == hipSuccess) e = copy_to_host(x, seg, used);
   if (e != hipSuccess) return hip_fail(x, e, "kmi_batch_moments");
   return KMI_OK;
 }

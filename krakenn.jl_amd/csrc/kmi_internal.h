@@ -6,19 +6,40 @@
 
 #include "kmi_common.h"
 
+namespace kmi {
+struct HostCopier;  // kmi_xfer.hip
+}
+
 struct kmi_ctx {
   int device = 0;
   hipStream_t stream = nullptr;
   std::string err;
-  double* partials = nullptr;  // 2048 groups × 3 values × (sum, error)
-  double* out = nullptr;       // 8 values
+  double* partials = nullptr;  // kRedPartials values, then the reductions' group counter
+  double* out = nullptr;       // 8 values in pinned host memory, written by the reductions
+  kmi::HostCopier* copier = nullptr;
 };
 
 namespace kmi {
 
+constexpr int kRedGroups = 2048;               // work-groups of a reduction at most
+constexpr int kRedPartials = kRedGroups * 3 * 2;  // groups × 3 values × (sum, error)
+
 // Record `msg` as the last error of `ctx` (or of the calling thread when ctx is NULL).
 int fail(kmi_ctx* ctx, int code, const std::string& msg);
 int hip_fail(kmi_ctx* ctx, hipError_t e, const char* what);
+
+// Host transfers on ctx->stream through the context's pinned buffers (kmi_xfer.hip).
+// copy_to_host returns when the data has arrived (and with it everything queued before);
+// copy_to_device when the host arrays may change, the device side in stream order.
+struct HostSeg {
+  void* host;
+  void* dev;
+  size_t bytes;
+};
+HostCopier* host_copier_create();
+void host_copier_destroy(HostCopier* c);
+hipError_t copy_to_host(kmi_ctx* ctx, const HostSeg* seg, int count);
+hipError_t copy_to_device(kmi_ctx* ctx, const HostSeg* seg, int count);
 
 hipError_t launch_step(int q, int st, int coll, bool th, bool bnd, bool nts, const StepArgs& a,
                        dim3 g, dim3 b, hipStream_t s);

@@ -1627,14 +1627,16 @@ int kmi_nn_param_count(const kmi_nn* N, int64_t* n) {
 int kmi_nn_get_params(kmi_nn* N, float* host) {
   if (!N || !host) return fail(nullptr, KMI_ERR_ARG, "kmi_nn_get_params: NULL argument");
   KMI_HIP(N->ctx, hipSetDevice(N->ctx->device));
-  KMI_HIP(N->ctx, hipMemcpy(host, N->w, N->nparam * 4, hipMemcpyDeviceToHost));
+  const HostSeg seg{host, N->w, size_t(N->nparam) * 4};
+  KMI_HIP(N->ctx, copy_to_host(N->ctx, &seg, 1));
   return KMI_OK;
 }
 
 int kmi_nn_set_params(kmi_nn* N, const float* host) {
   if (!N || !host) return fail(nullptr, KMI_ERR_ARG, "kmi_nn_set_params: NULL argument");
   KMI_HIP(N->ctx, hipSetDevice(N->ctx->device));
-  KMI_HIP(N->ctx, hipMemcpy(N->w, host, N->nparam * 4, hipMemcpyHostToDevice));
+  const HostSeg seg{const_cast<float*>(host), N->w, size_t(N->nparam) * 4};
+  KMI_HIP(N->ctx, copy_to_device(N->ctx, &seg, 1));
   hipLaunchKernelGGL(k_to_bf16, g1(N->nparam), dim3(256), 0, N->ctx->stream, N->w, N->nparam, N->wb);
   KMI_HIP(N->ctx, hipGetLastError());
   KMI_HIP(N->ctx, refresh_weight_copies(N, N->ctx->stream));
@@ -1657,8 +1659,8 @@ int kmi_nn_forward(kmi_nn* N, int32_t B, const float* x, float* y) {
   KMI_HIP(c, hipSetDevice(c->device));
   KMI_HIP(c, hipMemcpyAsync(N->x, x, (size_t)B * N->d.in_dim * 4, hipMemcpyHostToDevice, c->stream));
   if (int rc = nn_forward(N, B)) return rc;
-  KMI_HIP(c, hipMemcpyAsync(y, N->y, out_elems(N, B) * 4, hipMemcpyDeviceToHost, c->stream));
-  KMI_HIP(c, hipStreamSynchronize(c->stream));
+  const HostSeg seg{y, N->y, size_t(out_elems(N, B)) * 4};
+  KMI_HIP(c, copy_to_host(c, &seg, 1));
   return KMI_OK;
 }
 
@@ -1668,11 +1670,15 @@ int kmi_nn_loss_grad(kmi_nn* N, int32_t B, const float* x, const float* target, 
   kmi_ctx* c = N->ctx;
   KMI_HIP(c, hipSetDevice(c->device));
   KMI_HIP(c, hipMemcpyAsync(N->x, x, (size_t)B * N->d.in_dim * 4, hipMemcpyHostToDevice, c->stream));
-  KMI_HIP(c, hipMemcpyAsync(N->tgt, target, out_elems(N, B) * 4, hipMemcpyHostToDevice, c->stream));
+  const HostSeg in{const_cast<float*>(target), N->tgt, size_t(out_elems(N, B)) * 4};
+  KMI_HIP(c, copy_to_device(c, &in, 1));
   if (int rc = nn_forward(N, B)) return rc;
   if (int rc = nn_loss(N, B, loss)) return rc;
   if (int rc = nn_backward(N, B)) return rc;
-  if (grad) KMI_HIP(c, hipMemcpyAsync(grad, N->g, N->nparam * 4, hipMemcpyDeviceToHost, c->stream));
+  if (grad) {
+    const HostSeg out{grad, N->g, size_t(N->nparam) * 4};
+    KMI_HIP(c, copy_to_host(c, &out, 1));
+  }
   KMI_HIP(c, hipStreamSynchronize(c->stream));
   return KMI_OK;
 }
@@ -1699,8 +1705,10 @@ int kmi_nn_set_dataset(kmi_nn* N, int32_t n, const float* x, const float* y) {
   KMI_HIP(c, hipMalloc(&N->dsY, (size_t)n * dout * 4));
   KMI_HIP(c, hipMalloc(&N->perm_d, (size_t)n * 4));
   KMI_HIP(c, hipMalloc(&N->lhist, (size_t)n * 8));
-  KMI_HIP(c, hipMemcpy(N->dsX, x, (size_t)n * N->d.in_dim * 4, hipMemcpyHostToDevice));
-  KMI_HIP(c, hipMemcpy(N->dsY, y, (size_t)n * dout * 4, hipMemcpyHostToDevice));
+  const HostSeg seg[2] = {{const_cast<float*>(x), N->dsX, (size_t)n * N->d.in_dim * 4},
+                          {const_cast<float*>(y), N->dsY, (size_t)n * dout * 4}};
+  KMI_HIP(c, copy_to_device(c, seg, 2));
+  KMI_HIP(c, hipStreamSynchronize(c->stream));
   N->dsN = n;
   return KMI_OK;
 }

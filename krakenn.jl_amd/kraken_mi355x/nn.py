@@ -73,16 +73,22 @@ class WarmStartNet:
 
     def forward(self, x):
         x = _f32(x)
-        B = x.shape[0]
-        y = np.empty(self._out_shape(B), dtype=np.float32)
-        self._chk(L.load().kmi_nn_forward(self._h, B, _fp(x), _fp(y)))
+        y = np.empty(self._out_shape(x.shape[0]), dtype=np.float32)
+        self._forward_into(x, y)
         return y
 
+    def _forward_into(self, x, y):
+        self._chk(L.load().kmi_nn_forward(self._h, x.shape[0], _fp(x), _fp(y)))
+
     def predict(self, x):
-        """Forward in chunks of max_batch."""
+        """Forward in chunks of max_batch, each straight into its part of the result."""
         x = _f32(x)
-        outs = [self.forward(x[i:i + self.desc.max_batch]) for i in range(0, len(x), self.desc.max_batch)]
-        return np.concatenate(outs, axis=0)
+        if len(x) == 0:
+            raise ValueError("need at least one sample")
+        y = np.empty(self._out_shape(len(x)), dtype=np.float32)
+        for i in range(0, len(x), self.desc.max_batch):
+            self._forward_into(x[i:i + self.desc.max_batch], y[i:i + self.desc.max_batch])
+        return y
 
     def loss_grad(self, x, target, want_grad=True):
         x, t = _f32(x), _f32(target)
