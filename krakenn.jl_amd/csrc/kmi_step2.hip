@@ -239,16 +239,22 @@ KMI_DEV void pull_lds(R (&fp)[19], const R* A, const R* Bs, const R* Cs, const R
     constexpr int cx = Lat<19>::cx[q], cy = Lat<19>::cy[q], cz = Lat<19>::cz[q];
     constexpr int n = tb::group_index(q), o = Lat<19>::opp[q], no = tb::group_index(o);
     const int e = (ey - cy) * EXp + (ex - cx);
-    const R* src = (cz == 0 ? A : cz > 0 ? Bs : Cs) + n * NEp + e;
     if constexpr (BND && q != 0) {
+      const R* src = (cz == 0 ? A : cz > 0 ? Bs : Cs) + n * NEp + e;
       // one read at a selected address: written as branches, the bounced links put a divergent
       // branch on every link (run_cavity_3d's cube, F32S 256³ on 64×8 tiles, µs per step:
       // branches 382, selects 298, selects with the iterations off the z faces apart 279;
       // F64 128³ on 32×8 tiles: 117, 97, 88)
       const R* back = (cz == 0 ? A : cz > 0 ? Co : Bo) + no * NEp + own;
       src = tb::src_ok<q>(nb) ? src : back;
+      fp[q] = *src;
+    } else if constexpr (cz == 0) {
+      fp[q] = A[n * NEp + e];
+    } else if constexpr (cz > 0) {
+      fp[q] = Bs[n * NEp + e];
+    } else {
+      fp[q] = Cs[n * NEp + e];
     }
-    fp[q] = *src;
   });
   if constexpr (BND) tb::ladd_all<BND>(fp, a, nb);
 }
@@ -273,7 +279,7 @@ KMI_DEV void march_planes(const StepArgs& a, int lo, int hi, int nz, F&& iterate
 // NT threads per work-group, at least TX·TY: one per interior cell (a thread then evaluates
 // up to two extended cells in phase 1), or at least (TX+2)(TY+2), one per extended cell
 // (threads beyond TX·TY idle in phase 2).
-template <int ST, int COLL, int TX, int TY, int NT, bool NTS, int BND>
+template <int ST, int COLL, int TX, int TY, int NT, bool NTS>
 KMI_DEV void march2(const StepArgs& a, int zlen, int tx, int ty, int zc, typename Store<ST>::real* lds) {
   using S = Store<ST>;
   using E = typename S::elem;
@@ -282,12 +288,9 @@ KMI_DEV void march2(const StepArgs& a, int zlen, int tx, int ty, int zc, typenam
   static_assert(NT >= NI && NT % 64 == 0, "one thread per interior cell at least");
   constexpr int EPT = (NE + NT - 1) / NT;  // extended cells per work-item in phase 1
   constexpr unsigned ES = sizeof(E);
-  // walled lattices keep the c_z = −1 values of two planes (the cell's own plane feeds its
-  // bounced links), 29 values per extended cell
-  constexpr int NC = BND ? 2 : 1;
   R* const A = lds;            // c_z = 0:  [9][NE]
   R* const B = lds + 9 * NE;   // c_z = +1: [2 planes][5][NE]
-  R* const C = lds + 19 * NE;  // c_z = −1: [NC planes][5][NE]
+  R* const C = lds + 19 * NE;  // c_z = −1: [5][NE]
 
   const int nx = a.nx, ny = a.ny, nz = a.nz;
   const long long P = a.plane;
@@ -300,9 +303,136 @@ KMI_DEV void march2(const StepArgs& a, int zlen, int tx, int ty, int zc, typenam
   // Pull of the t populations of plane s for the extended cells this work-item owns.  With
   // FP32 arithmetic the pull for plane s+1 is issued before plane s is processed, so its HBM
   // latency overlaps the collisions, the barriers and the phase-2 stores of plane s; FP64
-  // and 1024-wide groups have no registers to spare for it.  Walled lattices: a link from
-  // beyond a wall reads the cell's own opposite population (halfway bounce-back, with the
-  // Ladd term of a moving wall); extended cells beyond a wall are never read and skipped.
+  // and 1024-wide groups have no registers to spare for it.
+  constexpr bool kPrefetch = sizeof(R) == 4 && (NT <= 512 || EPT == 1);
+  R nxt[EPT][19];
+  auto pull_plane = [&](int s) {
+    const int zs = tb::wrap(s, nz);
+    const int zm = tb::wrap(zs - 1, nz), zp = tb::wrap(zs + 1, nz);
+#pragma unroll
+    for (int r = 0; r < EPT; ++r) {
+      const int e = tid + r * NT;
+      if (e < NE) {
+        const int ex = e % EX, ey = e / EX;
+        const int gx = tb::wrap(x0 - 1 + ex, nx), gy = tb::wrap(y0 - 1 + ey, ny);
+        const int xm = tb::wrap(gx - 1, nx), xp = tb::wrap(gx + 1, nx);
+        const int ym = tb::wrap(gy - 1, ny), yp = tb::wrap(gy + 1, ny);
+        // byte offsets of the three source columns and of the nine source rows
+        const unsigned bx[3] = {unsigned(xm) * ES, unsigned(gx) * ES, unsigned(xp) * ES};
+        const int yy[3] = {ym, gy, yp}, zz[3] = {zm, zs, zp};
+        sfor<19>([&](auto qc) {
+          constexpr int q = decltype(qc)::value;
+          constexpr int cx = Lat<19>::cx[q], cy = Lat<19>::cy[q], cz = Lat<19>::cz[q];
+          const unsigned row = unsigned(nx) * unsigned(yy[1 - cy] + ny * zz[1 - cz]) * ES;
+          nxt[r][q] = Pops<ST>::ld(&tb::at(fi + q * P, row + bx[1 - cx]));
+        });
+      }
+    }
+  };
+  if constexpr (kPrefetch) pull_plane(z0 - 1);
+
+  // a plain loop, as in march3 (with the body in a lambda: another schedule, F16S 256³ on
+  // tile 12 181.5 instead of 177.4 µs per step)
+  for (int s = z0 - 1; s <= z1; ++s) {
+    const int u = s + 3;  // non-negative plane counter for the LDS ring slot
+    // ---- phase 1: t+1 on plane s, extended tile ----
+    if constexpr (!kPrefetch) pull_plane(s);
+    R cur[EPT][19];
+#pragma unroll
+    for (int r = 0; r < EPT; ++r)
+#pragma unroll
+      for (int q = 0; q < 19; ++q) cur[r][q] = nxt[r][q];
+    if constexpr (kPrefetch)
+      if (s < z1) pull_plane(s + 1);
+    R keep0[EPT][9], keepp[EPT][5];
+#pragma unroll
+    for (int r = 0; r < EPT; ++r) {
+      const int e = tid + r * NT;
+      if (e < NE) {
+        R fn[19];
+        const int gx = tb::wrap(x0 - 1 + e % EX, nx), gy = tb::wrap(y0 - 1 + e / EX, ny), gz = tb::wrap(s, nz);
+        update19<ST, COLL, 0>(cur[r], fn, a, gx, gy, gz);
+        sfor<19>([&](auto qc) {
+          constexpr int q = decltype(qc)::value;
+          constexpr int cz = Lat<19>::cz[q];
+          constexpr int n = tb::group_index(q);
+          const R v = Pops<ST>::round(fn[q]);
+          if constexpr (cz == 0) keep0[r][n] = v;
+          else if constexpr (cz > 0) keepp[r][n] = v;
+          else C[n * NE + e] = v;
+        });
+      }
+    }
+    __syncthreads();
+    // ---- phase 2: t+2 on plane s−1, interior tile ----
+    if (s >= z0 + 1 && tid < NI) {
+      const R* const Br = B + ((u - 2) & 1) * 5 * NE;  // c_z = +1 of plane s−2
+      const int ix = tid % TX, iy = tid / TX;
+      R fp[19], fn[19];
+      // the periodic pull written out: through pull_lds the allocator keeps 1–4 more
+      // VGPRs live, which takes the F16S 64×8 / 704-thread tile from 80 to 81 VGPRs and
+      // from two groups per CU to one (0.361 against 0.479 ms per launch)
+      sfor<19>([&](auto qc) {
+        constexpr int q = decltype(qc)::value;
+        constexpr int cx = Lat<19>::cx[q], cy = Lat<19>::cy[q], cz = Lat<19>::cz[q];
+        constexpr int n = tb::group_index(q);
+        const int e = (iy + 1 - cy) * EX + (ix + 1 - cx);
+        if constexpr (cz == 0) fp[q] = A[n * NE + e];
+        else if constexpr (cz > 0) fp[q] = Br[n * NE + e];
+        else fp[q] = C[n * NE + e];
+      });
+      update19<ST, COLL, 0>(fp, fn, a, x0 + ix, y0 + iy, s - 1);
+      const unsigned cell = (unsigned(x0 + ix) + unsigned(nx) * unsigned(y0 + iy + ny * (s - 1))) * ES;
+      sfor<19>([&](auto qc) {
+        constexpr int q = decltype(qc)::value;
+        Pops<ST>::template st<NTS>(tb::at(fo + q * P, cell), fn[q]);
+      });
+    }
+    __syncthreads();
+    // ---- phase 3: plane s's c_z = 0 and +1 populations into the slots phase 2 released ----
+    {
+      R* const Bw = B + (u & 1) * 5 * NE;
+#pragma unroll
+      for (int r = 0; r < EPT; ++r) {
+        const int e = tid + r * NT;
+        if (e < NE) {
+#pragma unroll
+          for (int n = 0; n < 9; ++n) A[n * NE + e] = keep0[r][n];
+#pragma unroll
+          for (int n = 0; n < 5; ++n) Bw[n * NE + e] = keepp[r][n];
+        }
+      }
+    }
+  }
+}
+
+// The walled two-step march.
+template <int ST, int COLL, int TX, int TY, int NT, bool NTS, int BND>
+KMI_DEV void march2_walled(const StepArgs& a, int zlen, int tx, int ty, int zc, typename Store<ST>::real* lds) {
+  using S = Store<ST>;
+  using E = typename S::elem;
+  using R = typename S::real;
+  constexpr int EX = TX + 2, EY = TY + 2, NE = EX * EY, NI = TX * TY;
+  static_assert(NT >= NI && NT % 64 == 0, "one thread per interior cell at least");
+  constexpr int EPT = (NE + NT - 1) / NT;  // extended cells per work-item in phase 1
+  constexpr unsigned ES = sizeof(E);
+  // the c_z = −1 values of two planes are kept (the cell's own plane feeds its bounced
+  // links), 29 values per extended cell
+  R* const A = lds;            // c_z = 0:  [9][NE]
+  R* const B = lds + 9 * NE;   // c_z = +1: [2 planes][5][NE]
+  R* const C = lds + 19 * NE;  // c_z = −1: [2 planes][5][NE]
+
+  const int nx = a.nx, ny = a.ny, nz = a.nz;
+  const long long P = a.plane;
+  const int x0 = tx * TX, y0 = ty * TY;
+  const int z0 = zc * zlen, z1 = min(z0 + zlen, nz);
+  const E* __restrict__ fi = static_cast<const E*>(a.fi);
+  E* __restrict__ fo = static_cast<E*>(a.fo);
+  const int tid = threadIdx.x;
+
+  // The pull as in march2; a link from beyond a wall reads the cell's own opposite population
+  // (halfway bounce-back, with the Ladd term of a moving wall); extended cells beyond a wall
+  // are never read and skipped.
   constexpr bool kPrefetch = sizeof(R) == 4 && (NT <= 512 || EPT == 1);
   R nxt[EPT][19];
   auto inside = [&](int s, int e, auto mc) {
@@ -330,8 +460,7 @@ KMI_DEV void march2(const StepArgs& a, int zlen, int tx, int ty, int zc, typenam
         // byte offsets of the three source columns and of the nine source rows
         const unsigned bx[3] = {unsigned(xm) * ES, unsigned(gx) * ES, unsigned(xp) * ES};
         const int yy[3] = {ym, gy, yp}, zz[3] = {zm, zs, zp};
-        tb::Nbr nb{};
-        if constexpr (M != 0) nb = tb::nbr<M>(a, gx, gy, zs);
+        const tb::Nbr nb = tb::nbr<M>(a, gx, gy, zs);
         const unsigned own = (unsigned(gx) + unsigned(nx) * unsigned(gy + ny * zs)) * ES;
         sfor<19>([&](auto qc) {
           constexpr int q = decltype(qc)::value;
@@ -339,7 +468,7 @@ KMI_DEV void march2(const StepArgs& a, int zlen, int tx, int ty, int zc, typenam
           const unsigned row = unsigned(nx) * unsigned(yy[1 - cy] + ny * zz[1 - cz]) * ES;
           const E* plane = fi + q * P;
           unsigned off = row + bx[1 - cx];
-          if constexpr (M != 0 && q != 0) {
+          if constexpr (q != 0) {
             const bool ok = tb::src_ok<q>(nb);
             plane = ok ? plane : fi + Lat<19>::opp[q] * P;
             off = ok ? off : own;
@@ -355,7 +484,7 @@ KMI_DEV void march2(const StepArgs& a, int zlen, int tx, int ty, int zc, typenam
   auto iterate = [&](int s, auto mc) {
     constexpr int M = decltype(mc)::value;
     const int u = s + 3;  // non-negative plane counter for the LDS ring slot
-    R* const Cw = C + (BND ? (u & 1) : 0) * 5 * NE;
+    R* const Cw = C + (u & 1) * 5 * NE;
     // ---- phase 1: t+1 on plane s, extended tile ----
     if constexpr (!kPrefetch) pull_plane(s, mc);
     R cur[EPT][19];
@@ -372,7 +501,7 @@ KMI_DEV void march2(const StepArgs& a, int zlen, int tx, int ty, int zc, typenam
       if (e < NE && inside(s, e, mc)) {
         R fn[19];
         const int gx = tb::wrap(x0 - 1 + e % EX, nx), gy = tb::wrap(y0 - 1 + e / EX, ny), gz = tb::wrap(s, nz);
-        if constexpr (M != 0) tb::ladd_all<M>(cur[r], a, tb::nbr<M>(a, gx, gy, gz));
+        tb::ladd_all<M>(cur[r], a, tb::nbr<M>(a, gx, gy, gz));
         update19<ST, COLL, M>(cur[r], fn, a, gx, gy, gz);
         sfor<19>([&](auto qc) {
           constexpr int q = decltype(qc)::value;
@@ -390,27 +519,11 @@ KMI_DEV void march2(const StepArgs& a, int zlen, int tx, int ty, int zc, typenam
     if (s >= z0 + 1 && tid < NI) {
       const R* const Br = B + ((u - 2) & 1) * 5 * NE;  // c_z = +1 of plane s−2
       const R* const Bo = B + ((u - 1) & 1) * 5 * NE;  // c_z = +1 of plane s−1 (own)
-      const R* const Co = C + (BND ? ((u - 1) & 1) : 0) * 5 * NE;  // c_z = −1 of plane s−1 (own)
+      const R* const Co = C + ((u - 1) & 1) * 5 * NE;  // c_z = −1 of plane s−1 (own)
       const int ix = tid % TX, iy = tid / TX;
-      tb::Nbr nb{};
-      if constexpr (M != 0) nb = tb::nbr<M>(a, x0 + ix, y0 + iy, s - 1);
+      const tb::Nbr nb = tb::nbr<M>(a, x0 + ix, y0 + iy, s - 1);
       R fp[19], fn[19];
-      if constexpr (BND == 0) {
-        // the periodic pull written out: through pull_lds the allocator keeps 1–4 more
-        // VGPRs live, which takes the F16S 64×8 / 704-thread tile from 80 to 81 VGPRs and
-        // from two groups per CU to one (0.361 against 0.479 ms per launch)
-        sfor<19>([&](auto qc) {
-          constexpr int q = decltype(qc)::value;
-          constexpr int cx = Lat<19>::cx[q], cy = Lat<19>::cy[q], cz = Lat<19>::cz[q];
-          constexpr int n = tb::group_index(q);
-          const int e = (iy + 1 - cy) * EX + (ix + 1 - cx);
-          if constexpr (cz == 0) fp[q] = A[n * NE + e];
-          else if constexpr (cz > 0) fp[q] = Br[n * NE + e];
-          else fp[q] = Cw[n * NE + e];
-        });
-      } else {
-        pull_lds<M>(fp, A, Br, Cw, Bo, Co, NE, EX, ix + 1, iy + 1, a, nb);
-      }
+      pull_lds<M>(fp, A, Br, Cw, Bo, Co, NE, EX, ix + 1, iy + 1, a, nb);
       update19<ST, COLL, M>(fp, fn, a, x0 + ix, y0 + iy, s - 1);
       const unsigned cell = (unsigned(x0 + ix) + unsigned(nx) * unsigned(y0 + iy + ny * (s - 1))) * ES;
       sfor<19>([&](auto qc) {
@@ -460,11 +573,12 @@ __global__ void __launch_bounds__(NT)
   const int tx = t % ntx, ty = (t / ntx) % nty, zc = t / (ntx * nty);
   if constexpr (BND >= 2) {
     if (tx >= inner.x && tx < inner.y && ty >= inner.z && ty < inner.w) {
-      march2<ST, COLL, TX, TY, NT, NTS, 1>(a, zlen, tx, ty, zc, lds);
+      march2_walled<ST, COLL, TX, TY, NT, NTS, 1>(a, zlen, tx, ty, zc, lds);
       return;
     }
   }
-  march2<ST, COLL, TX, TY, NT, NTS, BND>(a, zlen, tx, ty, zc, lds);
+  if constexpr (BND == 0) march2<ST, COLL, TX, TY, NT, NTS>(a, zlen, tx, ty, zc, lds);
+  else march2_walled<ST, COLL, TX, TY, NT, NTS, BND>(a, zlen, tx, ty, zc, lds);
 }
 
 // ---- three steps per launch ------------------------------------------------------------
@@ -502,7 +616,7 @@ constexpr int march3_lds_values(int TX, int TY) {
   return BND ? 29 * (n1 + n2) : 19 * n1 + 33 * n2;
 }
 
-template <int ST, int COLL, int TX, int TY, int NT, bool NTS, int BND>
+template <int ST, int COLL, int TX, int TY, int NT, bool NTS>
 KMI_DEV void march3(const StepArgs& a, int zlen, int tx, int ty, int zc, typename Store<ST>::real* lds) {
   using S = Store<ST>;
   using E = typename S::elem;
@@ -513,20 +627,188 @@ KMI_DEV void march3(const StepArgs& a, int zlen, int tx, int ty, int zc, typenam
   static_assert(NT >= NI && NT % 64 == 0, "one thread per interior cell at least");
   constexpr int EPT1 = (N1 + NT - 1) / NT, EPT2 = (N2 + NT - 1) / NT;
   constexpr unsigned ES = sizeof(E);
-  // Periodic lattices march with two barriers per plane (layout march3_lds_values<0>):
-  // level 1 keeps one slot per set (its c_z = +1 values are written one plane late, see
-  // below), level 2 two c_z = 0 slots and two c_z = +1 slots.  Walled lattices keep the
-  // three-barrier schedule and 24 values per cell and level, plus a second c_z = −1 plane
-  // (the cell's own plane feeds its bounced links).
-  constexpr bool TWO = BND == 0;
-  constexpr int NC = BND ? 2 : 1;  // c_z = −1 planes per level
-  R* const A1 = lds;                         // c_z = 0:  [9][N1]
-  R* const B1 = lds + 9 * N1;                // c_z = +1: [TWO ? 1 : 2 planes][5][N1]
-  R* const C1 = B1 + (TWO ? 5 : 10) * N1;    // c_z = −1: [NC planes][5][N1]
-  R* const L2 = C1 + 5 * NC * N1;
-  R* const A2 = L2;                          // [TWO ? 2 : 1 planes][9][N2]
-  R* const B2 = A2 + (TWO ? 18 : 9) * N2;    // [2][5][N2]
-  R* const C2 = B2 + 10 * N2;                // [NC][5][N2]
+  R* const A1 = lds;           // c_z = 0:  [9][N1]
+  R* const B1 = lds + 9 * N1;  // c_z = +1: [5][N1], written one plane late (see below)
+  R* const C1 = B1 + 5 * N1;   // c_z = −1: [5][N1]
+  R* const A2 = C1 + 5 * N1;   // [2 planes][9][N2]
+  R* const B2 = A2 + 18 * N2;  // [2][5][N2]
+  R* const C2 = B2 + 10 * N2;  // [5][N2]
+
+  const int nx = a.nx, ny = a.ny, nz = a.nz;
+  const long long P = a.plane;
+  const int x0 = tx * TX, y0 = ty * TY;
+  const int z0 = zc * zlen, z1 = min(z0 + zlen, nz);
+  const E* __restrict__ fi = static_cast<const E*>(a.fi);
+  E* __restrict__ fo = static_cast<E*>(a.fo);
+  const int tid = threadIdx.x;
+
+  constexpr bool kPrefetch = sizeof(R) == 4 && (NT <= 512 || EPT1 == 1);
+  R nxt[EPT1][19];
+  auto pull_plane = [&](int s) {
+    const int zs = tb::wrap(s, nz);
+    const int zm = tb::wrap(zs - 1, nz), zp = tb::wrap(zs + 1, nz);
+#pragma unroll
+    for (int r = 0; r < EPT1; ++r) {
+      const int e = tid + r * NT;
+      if (e < N1) {
+        const int ex = e % E1X, ey = e / E1X;
+        const int gx = tb::wrap(x0 - 2 + ex, nx), gy = tb::wrap(y0 - 2 + ey, ny);
+        const int xm = tb::wrap(gx - 1, nx), xp = tb::wrap(gx + 1, nx);
+        const int ym = tb::wrap(gy - 1, ny), yp = tb::wrap(gy + 1, ny);
+        const unsigned bx[3] = {unsigned(xm) * ES, unsigned(gx) * ES, unsigned(xp) * ES};
+        const int yy[3] = {ym, gy, yp}, zz[3] = {zm, zs, zp};
+        sfor<19>([&](auto qc) {
+          constexpr int q = decltype(qc)::value;
+          constexpr int cx = Lat<19>::cx[q], cy = Lat<19>::cy[q], cz = Lat<19>::cz[q];
+          const unsigned row = unsigned(nx) * unsigned(yy[1 - cy] + ny * zz[1 - cz]) * ES;
+          nxt[r][q] = Pops<ST>::ld(&tb::at(fi + q * P, row + bx[1 - cx]));
+        });
+      }
+    }
+  };
+  if constexpr (kPrefetch) pull_plane(z0 - 2);
+  // the c_z = +1 values of the previous plane, held one plane longer
+  R k1q[EPT1][5] = {}, k2q[EPT2][5] = {};
+
+  // a plain loop: with the body in a lambda the prefetched cell was copied in the registers
+  // at the head of every plane (19 more moves in 829 instructions; F32S 256³ on tile 11
+  // 233.7 instead of 224.5 µs per step)
+  for (int s = z0 - 2; s <= z1 + 1; ++s) {
+    const int u = s + 4;  // non-negative plane counter for the ring slots
+    // ---- P1: t+1 on plane s, level-1 tile ----
+    if constexpr (!kPrefetch) pull_plane(s);
+    R cur[EPT1][19];
+#pragma unroll
+    for (int r = 0; r < EPT1; ++r)
+#pragma unroll
+      for (int q = 0; q < 19; ++q) cur[r][q] = nxt[r][q];
+    if constexpr (kPrefetch)
+      if (s <= z1) pull_plane(s + 1);
+    R k1z[EPT1][9], k1p[EPT1][5];
+#pragma unroll
+    for (int r = 0; r < EPT1; ++r) {
+      const int e = tid + r * NT;
+      if (e < N1) {
+        R fn[19];
+        const int gx = tb::wrap(x0 - 2 + e % E1X, nx), gy = tb::wrap(y0 - 2 + e / E1X, ny), gz = tb::wrap(s, nz);
+        update19<ST, COLL, 0>(cur[r], fn, a, gx, gy, gz);
+        sfor<19>([&](auto qc) {
+          constexpr int q = decltype(qc)::value;
+          constexpr int cz = Lat<19>::cz[q];
+          constexpr int n = tb::group_index(q);
+          const R v = Pops<ST>::round(fn[q]);
+          if constexpr (cz == 0) k1z[r][n] = v;
+          else if constexpr (cz > 0) k1p[r][n] = v;
+          else C1[n * N1 + e] = v;
+        });
+      }
+    }
+    __syncthreads();
+    // ---- P2: t+2 on plane s−1, level-2 tile ----
+    R k2z[EPT2][9], k2p[EPT2][5];
+    if (s >= z0) {
+#pragma unroll
+      for (int r = 0; r < EPT2; ++r) {
+        const int e = tid + r * NT;
+        if (e < N2) {
+          const int ex = e % E2X, ey = e / E2X;
+          const int gx = tb::wrap(x0 - 1 + ex, nx), gy = tb::wrap(y0 - 1 + ey, ny), gz = tb::wrap(s - 1, nz);
+          R fp[19], fn[19];
+          pull_lds<0>(fp, A1, B1, C1, B1, C1, N1, E1X, ex + 1, ey + 1, a, tb::Nbr{});
+          update19<ST, COLL, 0>(fp, fn, a, gx, gy, gz);
+          sfor<19>([&](auto qc) {
+            constexpr int q = decltype(qc)::value;
+            constexpr int cz = Lat<19>::cz[q];
+            constexpr int n = tb::group_index(q);
+            const R v = Pops<ST>::round(fn[q]);
+            if constexpr (cz == 0) k2z[r][n] = v;
+            else if constexpr (cz > 0) k2p[r][n] = v;
+            else C2[n * N2 + e] = v;
+          });
+        }
+      }
+    }
+    __syncthreads();
+    // ---- P3: t+3 on plane s−2, interior ----
+    if (s >= z0 + 2 && tid < NI) {
+      // These waves also evaluate the next plane's P1 before the next
+      // barrier, so their P3 issues ahead of the waves that already moved on to it (wave
+      // priority only; 0.8 % shorter launches for 64×8 / 832 threads, measured same-box).
+      __builtin_amdgcn_s_setprio(2);
+      const R* const A2r = A2 + ((u - 2) & 1) * 9 * N2;  // c_z = 0 of plane s−2
+      const R* const B2r = B2 + ((u - 3) & 1) * 5 * N2;  // c_z = +1 of plane s−3
+      const int ix = tid % TX, iy = tid / TX;
+      R fp[19], fn[19];
+      pull_lds<0>(fp, A2r, B2r, C2, B2r, C2, N2, E2X, ix + 1, iy + 1, a, tb::Nbr{});
+      update19<ST, COLL, 0>(fp, fn, a, x0 + ix, y0 + iy, s - 2);
+      const unsigned cell = (unsigned(x0 + ix) + unsigned(nx) * unsigned(y0 + iy + ny * (s - 2))) * ES;
+      sfor<19>([&](auto qc) {
+        constexpr int q = decltype(qc)::value;
+        Pops<ST>::template st<NTS>(tb::at(fo + q * P, cell), fn[q]);
+      });
+      __builtin_amdgcn_s_setprio(0);
+    }
+    // The values kept in P1 and P2 go to LDS after P3 (so P3, which the next barrier
+    // waits for, starts at once), into slots nobody reads until the next plane's P2
+    // (level 1) and P3 (level 2): level 1 takes plane s's c_z = 0 values and plane s−1's
+    // c_z = +1 values (P2 has read plane s−2's from that slot); level 2 takes plane s−1's
+    // c_z = 0 values and plane s−2's c_z = +1 values, in the slots P3 does not read.  The
+    // next plane's P1 writes only L1.C, whose reader (P2) finished before the last
+    // barrier, so no third barrier is needed: threads without a P3 cell go straight on to
+    // the next plane's P1.
+#pragma unroll
+    for (int r = 0; r < EPT1; ++r) {
+      const int e = tid + r * NT;
+      if (e < N1) {
+#pragma unroll
+        for (int n = 0; n < 9; ++n) A1[n * N1 + e] = k1z[r][n];
+#pragma unroll
+        for (int n = 0; n < 5; ++n) {
+          B1[n * N1 + e] = k1q[r][n];
+          k1q[r][n] = k1p[r][n];
+        }
+      }
+    }
+    if (s >= z0) {
+      R* const A2w = A2 + ((u - 1) & 1) * 9 * N2;  // plane s−1
+      R* const B2w = B2 + ((u - 2) & 1) * 5 * N2;  // plane s−2
+#pragma unroll
+      for (int r = 0; r < EPT2; ++r) {
+        const int e = tid + r * NT;
+        if (e < N2) {
+#pragma unroll
+          for (int n = 0; n < 9; ++n) A2w[n * N2 + e] = k2z[r][n];
+#pragma unroll
+          for (int n = 0; n < 5; ++n) {
+            B2w[n * N2 + e] = k2q[r][n];
+            k2q[r][n] = k2p[r][n];
+          }
+        }
+      }
+    }
+  }
+}
+
+// The walled march: see the schedule above.
+template <int ST, int COLL, int TX, int TY, int NT, bool NTS, int BND>
+KMI_DEV void march3_walled(const StepArgs& a, int zlen, int tx, int ty, int zc, typename Store<ST>::real* lds) {
+  using S = Store<ST>;
+  using E = typename S::elem;
+  using R = typename S::real;
+  constexpr int E1X = TX + 4, E1Y = TY + 4, N1 = E1X * E1Y;  // level 1 (t+1)
+  constexpr int E2X = TX + 2, E2Y = TY + 2, N2 = E2X * E2Y;  // level 2 (t+2)
+  constexpr int NI = TX * TY;
+  static_assert(NT >= NI && NT % 64 == 0, "one thread per interior cell at least");
+  constexpr int EPT1 = (N1 + NT - 1) / NT, EPT2 = (N2 + NT - 1) / NT;
+  constexpr unsigned ES = sizeof(E);
+  // three barriers per plane, 24 values per cell and level, and a second c_z = −1 plane (the
+  // cell's own plane feeds its bounced links)
+  R* const A1 = lds;            // c_z = 0:  [9][N1]
+  R* const B1 = lds + 9 * N1;   // c_z = +1: [2 planes][5][N1]
+  R* const C1 = B1 + 10 * N1;   // c_z = −1: [2][5][N1]
+  R* const A2 = C1 + 10 * N1;   // [9][N2]
+  R* const B2 = A2 + 9 * N2;    // [2][5][N2]
+  R* const C2 = B2 + 10 * N2;   // [2][5][N2]
 
   const int nx = a.nx, ny = a.ny, nz = a.nz;
   const long long P = a.plane;
@@ -560,8 +842,7 @@ KMI_DEV void march3(const StepArgs& a, int zlen, int tx, int ty, int zc, typenam
         const int ym = tb::wrap(gy - 1, ny), yp = tb::wrap(gy + 1, ny);
         const unsigned bx[3] = {unsigned(xm) * ES, unsigned(gx) * ES, unsigned(xp) * ES};
         const int yy[3] = {ym, gy, yp}, zz[3] = {zm, zs, zp};
-        tb::Nbr nb{};
-        if constexpr (M != 0) nb = tb::nbr<M>(a, gx, gy, zs);
+        const tb::Nbr nb = tb::nbr<M>(a, gx, gy, zs);
         const unsigned own = (unsigned(gx) + unsigned(nx) * unsigned(gy + ny * zs)) * ES;
         sfor<19>([&](auto qc) {
           constexpr int q = decltype(qc)::value;
@@ -569,7 +850,7 @@ KMI_DEV void march3(const StepArgs& a, int zlen, int tx, int ty, int zc, typenam
           const unsigned row = unsigned(nx) * unsigned(yy[1 - cy] + ny * zz[1 - cz]) * ES;
           const E* plane = fi + q * P;
           unsigned off = row + bx[1 - cx];
-          if constexpr (M != 0 && q != 0) {
+          if constexpr (q != 0) {
             const bool ok = tb::src_ok<q>(nb);
             plane = ok ? plane : fi + Lat<19>::opp[q] * P;
             off = ok ? off : own;
@@ -580,15 +861,13 @@ KMI_DEV void march3(const StepArgs& a, int zlen, int tx, int ty, int zc, typenam
     }
   };
   if constexpr (kPrefetch) pull_plane(z0 - 2, std::integral_constant<int, BND>{});
-  // two-barrier schedule: the c_z = +1 values of the previous plane, held one plane longer
-  R k1q[TWO ? EPT1 : 1][5] = {}, k2q[TWO ? EPT2 : 1][5] = {};
 
   // One plane of the march; M: the mode of its cells (BND, or its form off the z faces).
   auto iterate = [&](int s, auto mc) {
     constexpr int M = decltype(mc)::value;
     const int u = s + 4;  // non-negative plane counter for the ring slots
-    R* const C1w = C1 + (BND ? (u & 1) : 0) * 5 * N1;        // c_z = −1, level 1, plane s
-    R* const C2w = C2 + (BND ? ((u - 1) & 1) : 0) * 5 * N2;  // c_z = −1, level 2, plane s−1
+    R* const C1w = C1 + (u & 1) * 5 * N1;        // c_z = −1, level 1, plane s
+    R* const C2w = C2 + ((u - 1) & 1) * 5 * N2;  // c_z = −1, level 2, plane s−1
     // ---- P1: t+1 on plane s, level-1 tile ----
     if constexpr (!kPrefetch) pull_plane(s, mc);
     R cur[EPT1][19];
@@ -605,7 +884,7 @@ KMI_DEV void march3(const StepArgs& a, int zlen, int tx, int ty, int zc, typenam
       if (e < N1 && inside(x0 - 2 + e % E1X, y0 - 2 + e / E1X, s, mc)) {
         R fn[19];
         const int gx = tb::wrap(x0 - 2 + e % E1X, nx), gy = tb::wrap(y0 - 2 + e / E1X, ny), gz = tb::wrap(s, nz);
-        if constexpr (M != 0) tb::ladd_all<M>(cur[r], a, tb::nbr<M>(a, gx, gy, gz));
+        tb::ladd_all<M>(cur[r], a, tb::nbr<M>(a, gx, gy, gz));
         update19<ST, COLL, M>(cur[r], fn, a, gx, gy, gz);
         sfor<19>([&](auto qc) {
           constexpr int q = decltype(qc)::value;
@@ -622,17 +901,16 @@ KMI_DEV void march3(const StepArgs& a, int zlen, int tx, int ty, int zc, typenam
     // ---- P2: t+2 on plane s−1, level-2 tile ----
     R k2z[EPT2][9], k2p[EPT2][5];
     if (s >= z0) {
-      const R* const B1r = B1 + (TWO ? 0 : ((u - 2) & 1) * 5 * N1);  // c_z = +1 of plane s−2
-      const R* const B1o = B1 + ((u - 1) & 1) * 5 * N1;  // c_z = +1 of plane s−1 (own; walled only)
-      const R* const C1o = C1 + (BND ? ((u - 1) & 1) : 0) * 5 * N1;  // c_z = −1 of plane s−1 (own)
+      const R* const B1r = B1 + ((u - 2) & 1) * 5 * N1;  // c_z = +1 of plane s−2
+      const R* const B1o = B1 + ((u - 1) & 1) * 5 * N1;  // c_z = +1 of plane s−1 (own)
+      const R* const C1o = C1 + ((u - 1) & 1) * 5 * N1;  // c_z = −1 of plane s−1 (own)
 #pragma unroll
       for (int r = 0; r < EPT2; ++r) {
         const int e = tid + r * NT;
         if (e < N2 && inside(x0 - 1 + e % E2X, y0 - 1 + e / E2X, s - 1, mc)) {
           const int ex = e % E2X, ey = e / E2X;
           const int gx = tb::wrap(x0 - 1 + ex, nx), gy = tb::wrap(y0 - 1 + ey, ny), gz = tb::wrap(s - 1, nz);
-          tb::Nbr nb{};
-          if constexpr (M != 0) nb = tb::nbr<M>(a, gx, gy, gz);
+          const tb::Nbr nb = tb::nbr<M>(a, gx, gy, gz);
           R fp[19], fn[19];
           pull_lds<M>(fp, A1, B1r, C1w, B1o, C1o, N1, E1X, ex + 1, ey + 1, a, nb);
           update19<ST, COLL, M>(fp, fn, a, gx, gy, gz);
@@ -649,96 +927,47 @@ KMI_DEV void march3(const StepArgs& a, int zlen, int tx, int ty, int zc, typenam
       }
     }
     __syncthreads();
-    // ---- P3: t+3 on plane s−2, interior (walled: then the P1 values into level 1) ----
+    // ---- P3: t+3 on plane s−2, interior; then the P1 values into level 1 ----
     if (s >= z0 + 2 && tid < NI) {
-      // Two-barrier schedule: these waves also evaluate the next plane's P1 before the next
-      // barrier, so their P3 issues ahead of the waves that already moved on to it (wave
-      // priority only; 0.8 % shorter launches for 64×8 / 832 threads, measured same-box).
-      if constexpr (TWO) __builtin_amdgcn_s_setprio(2);
-      const R* const A2r = A2 + (TWO ? ((u - 2) & 1) * 9 * N2 : 0);  // c_z = 0 of plane s−2
       const R* const B2r = B2 + ((u - 3) & 1) * 5 * N2;  // c_z = +1 of plane s−3
       const R* const B2o = B2 + ((u - 2) & 1) * 5 * N2;  // c_z = +1 of plane s−2 (own)
-      const R* const C2o = C2 + (BND ? ((u - 2) & 1) : 0) * 5 * N2;  // c_z = −1 of plane s−2 (own)
+      const R* const C2o = C2 + ((u - 2) & 1) * 5 * N2;  // c_z = −1 of plane s−2 (own)
       const int ix = tid % TX, iy = tid / TX;
-      tb::Nbr nb{};
-      if constexpr (M != 0) nb = tb::nbr<M>(a, x0 + ix, y0 + iy, s - 2);
+      const tb::Nbr nb = tb::nbr<M>(a, x0 + ix, y0 + iy, s - 2);
       R fp[19], fn[19];
-      pull_lds<M>(fp, A2r, B2r, C2w, B2o, C2o, N2, E2X, ix + 1, iy + 1, a, nb);
+      pull_lds<M>(fp, A2, B2r, C2w, B2o, C2o, N2, E2X, ix + 1, iy + 1, a, nb);
       update19<ST, COLL, M>(fp, fn, a, x0 + ix, y0 + iy, s - 2);
       const unsigned cell = (unsigned(x0 + ix) + unsigned(nx) * unsigned(y0 + iy + ny * (s - 2))) * ES;
       sfor<19>([&](auto qc) {
         constexpr int q = decltype(qc)::value;
         Pops<ST>::template st<NTS>(tb::at(fo + q * P, cell), fn[q]);
       });
-      if constexpr (TWO) __builtin_amdgcn_s_setprio(0);
     }
-    if constexpr (TWO) {
-      // The values kept in P1 and P2 go to LDS after P3 (so P3, which the next barrier
-      // waits for, starts at once), into slots nobody reads until the next plane's P2
-      // (level 1) and P3 (level 2): level 1 takes plane s's c_z = 0 values and plane s−1's
-      // c_z = +1 values (P2 has read plane s−2's from that slot); level 2 takes plane s−1's
-      // c_z = 0 values and plane s−2's c_z = +1 values, in the slots P3 does not read.  The
-      // next plane's P1 writes only L1.C, whose reader (P2) finished before the last
-      // barrier, so no third barrier is needed: threads without a P3 cell go straight on to
-      // the next plane's P1.
+    {
+      R* const B1w = B1 + (u & 1) * 5 * N1;
 #pragma unroll
       for (int r = 0; r < EPT1; ++r) {
         const int e = tid + r * NT;
-        if (e < N1) {
+        if (e < N1 && inside(x0 - 2 + e % E1X, y0 - 2 + e / E1X, s, mc)) {
 #pragma unroll
           for (int n = 0; n < 9; ++n) A1[n * N1 + e] = k1z[r][n];
 #pragma unroll
-          for (int n = 0; n < 5; ++n) {
-            B1[n * N1 + e] = k1q[r][n];
-            k1q[r][n] = k1p[r][n];
-          }
-        }
-      }
-      if (s >= z0) {
-        R* const A2w = A2 + ((u - 1) & 1) * 9 * N2;  // plane s−1
-        R* const B2w = B2 + ((u - 2) & 1) * 5 * N2;  // plane s−2
-#pragma unroll
-        for (int r = 0; r < EPT2; ++r) {
-          const int e = tid + r * NT;
-          if (e < N2) {
-#pragma unroll
-            for (int n = 0; n < 9; ++n) A2w[n * N2 + e] = k2z[r][n];
-#pragma unroll
-            for (int n = 0; n < 5; ++n) {
-              B2w[n * N2 + e] = k2q[r][n];
-              k2q[r][n] = k2p[r][n];
-            }
-          }
+          for (int n = 0; n < 5; ++n) B1w[n * N1 + e] = k1p[r][n];
         }
       }
     }
-    if constexpr (!TWO) {
-      {
-        R* const B1w = B1 + (u & 1) * 5 * N1;
+    __syncthreads();
+    // ---- P4: the P2 values (plane s−1) into level 2 ----
+    if (s >= z0) {
+      R* const B2w = B2 + ((u - 1) & 1) * 5 * N2;
 #pragma unroll
-        for (int r = 0; r < EPT1; ++r) {
-          const int e = tid + r * NT;
-          if (e < N1 && inside(x0 - 2 + e % E1X, y0 - 2 + e / E1X, s, mc)) {
+      for (int r = 0; r < EPT2; ++r) {
+        const int e = tid + r * NT;
+        if (e < N2 && inside(x0 - 1 + e % E2X, y0 - 1 + e / E2X, s - 1, mc)) {
 #pragma unroll
-            for (int n = 0; n < 9; ++n) A1[n * N1 + e] = k1z[r][n];
+          for (int n = 0; n < 9; ++n) A2[n * N2 + e] = k2z[r][n];
 #pragma unroll
-            for (int n = 0; n < 5; ++n) B1w[n * N1 + e] = k1p[r][n];
-          }
-        }
-      }
-      __syncthreads();
-      // ---- P4: the P2 values (plane s−1) into level 2 ----
-      if (s >= z0) {
-        R* const B2w = B2 + ((u - 1) & 1) * 5 * N2;
-#pragma unroll
-        for (int r = 0; r < EPT2; ++r) {
-          const int e = tid + r * NT;
-          if (e < N2 && inside(x0 - 1 + e % E2X, y0 - 1 + e / E2X, s - 1, mc)) {
-#pragma unroll
-            for (int n = 0; n < 9; ++n) A2[n * N2 + e] = k2z[r][n];
-#pragma unroll
-            for (int n = 0; n < 5; ++n) B2w[n * N2 + e] = k2p[r][n];
-          }
+          for (int n = 0; n < 5; ++n) B2w[n * N2 + e] = k2p[r][n];
         }
       }
     }
@@ -764,11 +993,12 @@ __global__ void __launch_bounds__(NT)
   const int tx = t % ntx, ty = (t / ntx) % nty, zc = t / (ntx * nty);
   if constexpr (BND >= 2) {
     if (tx >= inner.x && tx < inner.y && ty >= inner.z && ty < inner.w) {
-      march3<ST, COLL, TX, TY, NT, NTS, 1>(a, zlen, tx, ty, zc, lds);
+      march3_walled<ST, COLL, TX, TY, NT, NTS, 1>(a, zlen, tx, ty, zc, lds);
       return;
     }
   }
-  march3<ST, COLL, TX, TY, NT, NTS, BND>(a, zlen, tx, ty, zc, lds);
+  if constexpr (BND == 0) march3<ST, COLL, TX, TY, NT, NTS>(a, zlen, tx, ty, zc, lds);
+  else march3_walled<ST, COLL, TX, TY, NT, NTS, BND>(a, zlen, tx, ty, zc, lds);
 }
 
 // ---- dispatch ---------------------------------------------------------------------------
