@@ -357,7 +357,11 @@ int kmi_lattice_get_launch(const kmi_lattice* lat, int32_t* bx, int32_t* by, int
  * of a lattice of at least 160,000 cells without mask, forcing or thermal populations marches
  * strips of columns in registers instead (four steps as well).
  * Results are bit-identical to single-step launches; step counts that are not a multiple
- * of the span end with single steps. */
+ * of the span end with single steps.
+ * A D3Q19 lattice on which no launch was set (here, by kmi_lattice_set_launch or by
+ * kmi_lattice_autotune) takes the multi-step launch expected to be fastest for its sizes and
+ * storage, of any x-y extent of at least a tile, or single steps where those are faster;
+ * kmi_lattice_get_temporal reports tile 0 for it.  set_temporal(0) asks for single steps. */
 int kmi_lattice_set_temporal(kmi_lattice* lat, int32_t tile, int32_t zchunks);
 int kmi_lattice_get_temporal(const kmi_lattice* lat, int32_t* tile, int32_t* zchunks);
 /* Time every candidate shape × store policy (and two-step variant, where it applies) on

@@ -44,6 +44,9 @@ struct kmi_lattice {
   bool bnd = true;
   int bx = 0, by = 1, nts = 0;  // launch shape and store policy (0: not chosen yet)
   int tb_tile = 0, tb_zchunks = 1;  // two-step launches (0: off), see kmi_step2.hip
+  // D3Q19: tb_tile and tb_zchunks are the lattice's own choice (step2_plan, any x–y extent),
+  // made again before each run; off once a launch is set by the user or the tuner
+  bool tb_auto = false;
   // work-group → tile table of the walled multi-step launch (device), built for order_key
   int* order = nullptr;
   size_t order_cap = 0;
@@ -409,7 +412,7 @@ static void default_geometry(kmi_lattice* L) {
 // mask; no forcing, no cut links) on the walled tiles (12, 14; 9 except FP64; not F16S).  D2Q9 (k_step_tb2d):
 // no cut links, faces periodic / wall / moving wall / constant Zou–He only (thermal lattices
 // included), and a lattice of at least the tile plus its ring on each axis.
-static bool tb_eligible(const kmi_lattice* L, int tile) {
+static bool tb_eligible(const kmi_lattice* L, int tile, bool any_extent = false) {
   if (L->Q == 9) {
     int TW, TH, K;
     if (!tb2d_variant(tile, TW, TH, K) || !L->cut_cells.empty()) return false;
@@ -421,8 +424,9 @@ static bool tb_eligible(const kmi_lattice* L, int tile) {
   int TX, TY;
   if (!step2_tile(tile, L->desc.storage, TX, TY)) return false;
   if (L->Q != 19 || L->desc.thermal || (L->desc.collision != KMI_BGK && L->desc.collision != KMI_TRT) ||
-      L->desc.nx % TX != 0 || L->desc.ny % TY != 0 || L->args.nz < 4)
+      L->desc.nx < TX || L->desc.ny < TY || L->args.nz < 4)
     return false;
+  if (!any_extent && (L->desc.nx % TX != 0 || L->desc.ny % TY != 0)) return false;
   if (!L->bnd) return true;
   // walled lattices: halfway / moving-wall bounce-back, constant Zou–He faces and solid masks,
   // without forcing or cut links, on the walled tiles
@@ -445,7 +449,7 @@ static bool march_applies(const kmi_lattice* L) {
 
 // Steps advanced by one launch.
 static int launch_span(const kmi_lattice* L) {
-  if (!L->tb_tile || !tb_eligible(L, L->tb_tile)) return 1;
+  if (!L->tb_tile || !tb_eligible(L, L->tb_tile, L->tb_auto)) return 1;
   if (L->Q == 9) {
     int TW, TH, K;
     tb2d_variant(L->tb_tile, TW, TH, K);
@@ -469,7 +473,7 @@ static int launch_one(kmi_lattice* L, hipStream_t s, bool multi = false) {
   a.mask = L->mask;
   // the table only for the tile and z-split it was built for (any other launch keeps the
   // default order, which covers every tile as well)
-  a.tile_order = multi && L->bnd && L->Q == 19 && L->order && L->order_key[0] == L->tb_tile &&
+  a.tile_order = multi && L->bnd && L->Q == 19 && !L->tb_auto && L->order && L->order_key[0] == L->tb_tile &&
                          L->order_key[1] == L->tb_zchunks
                      ? L->order
                      : nullptr;
@@ -501,7 +505,7 @@ static void drop_graphs(kmi_lattice* L) {
 // tile and z-split, rebuilt when those change — before any graph capture, since the upload
 // is an ordinary copy on the lattice stream.
 static int refresh_tile_order(kmi_lattice* L) {
-  if (!(L->bnd && L->Q == 19 && L->tb_tile)) return KMI_OK;
+  if (!(L->bnd && L->Q == 19 && L->tb_tile) || L->tb_auto) return KMI_OK;
   if (L->order && L->order_key[0] == L->tb_tile && L->order_key[1] == L->tb_zchunks) return KMI_OK;
   std::vector<int> h;
   walled_tile_order(L->args, L->tb_tile, L->tb_zchunks, h);
@@ -524,9 +528,21 @@ static int refresh_tile_order(kmi_lattice* L) {
   return KMI_OK;
 }
 
+// The lattice's own multi-step launch (tb_auto); faces, masks and cut links may have changed
+// since the last run.
+static void refresh_plan(kmi_lattice* L) {
+  int tile = 0, zchunks = 1;
+  if (!step2_plan(L->desc.storage, L->bnd, L->args, tile, zchunks) || !tb_eligible(L, tile, true)) tile = 0, zchunks = 1;
+  if (tile == L->tb_tile && zchunks == L->tb_zchunks) return;
+  drop_graphs(L);
+  L->tb_tile = tile;
+  L->tb_zchunks = zchunks;
+}
+
 static int run_steps(kmi_lattice* L, int64_t n) {
   kmi_ctx* c = L->ctx;
   hipStream_t s = c->stream;
+  if (L->tb_auto && n > 1) refresh_plan(L);
   if (int rc = refresh_tile_order(L); rc != KMI_OK) return rc;
   const int span = launch_span(L);
   const int gsteps = graph_steps(L);
@@ -638,6 +654,7 @@ int kmi_lattice_create(kmi_ctx* ctx, const kmi_desc* desc, kmi_lattice** out) {
   }
   build_args(L);
   default_geometry(L);
+  L->tb_auto = L->Q == 19;
   // rest equilibrium f = w_q, g = w_q T_ref (initialize_2d/3d, basic.jl:64-70)
   int rc = kmi_init_equilibrium(L, nullptr, nullptr, nullptr, nullptr);
   if (rc == KMI_OK && desc->thermal) rc = kmi_init_temperature(L, nullptr);
@@ -1225,6 +1242,7 @@ int kmi_lattice_set_launch(kmi_lattice* L, int32_t bx, int32_t by, int32_t nonte
   KMI_HIP(L->ctx, hipStreamSynchronize(L->ctx->stream));
   drop_graphs(L);
   set_geometry(L, bx, by, nontemporal ? 1 : 0);
+  if (L->tb_auto) L->tb_auto = false, L->tb_tile = 0, L->tb_zchunks = 1;  // the shape asked for
   return KMI_OK;
 }
 
@@ -1258,6 +1276,7 @@ int kmi_lattice_set_temporal(kmi_lattice* L, int32_t tile, int32_t zchunks) {
   KMI_HIP(L->ctx, hipSetDevice(L->ctx->device));
   KMI_HIP(L->ctx, hipStreamSynchronize(L->ctx->stream));
   drop_graphs(L);
+  L->tb_auto = false;
   L->tb_tile = tile;
   L->tb_zchunks = tile ? zchunks : 1;
   return KMI_OK;
@@ -1266,8 +1285,8 @@ int kmi_lattice_set_temporal(kmi_lattice* L, int32_t tile, int32_t zchunks) {
 int kmi_lattice_get_temporal(const kmi_lattice* L, int32_t* tile, int32_t* zchunks) {
   if (!L || !tile || !zchunks)
     return fail(nullptr, KMI_ERR_ARG, "kmi_lattice_get_temporal: NULL argument");
-  *tile = L->tb_tile;
-  *zchunks = L->tb_zchunks;
+  *tile = L->tb_auto ? 0 : L->tb_tile;  // 0: none chosen
+  *zchunks = L->tb_auto ? 1 : L->tb_zchunks;
   return KMI_OK;
 }
 
@@ -1314,7 +1333,9 @@ int kmi_lattice_autotune(kmi_lattice* L, int64_t steps_per_trial, double* best_m
   const int shapes[][2] = {{256, 1}, {128, 1}, {128, 2}, {64, 1}, {64, 2}, {64, 4}, {32, 2},
                            {32, 4}, {32, 8}, {16, 4}, {16, 8}, {16, 16}};
   double best = 1e300;
-  int bb[5] = {L->bx, L->by, L->nts, L->tb_tile, L->tb_zchunks};
+  const bool auto0 = L->tb_auto;
+  int bb[5] = {L->bx, L->by, L->nts, auto0 ? 0 : L->tb_tile, auto0 ? 1 : L->tb_zchunks};
+  L->tb_auto = false;
   L->tb_tile = 0;
   for (const auto& sh : shapes) {
     if (e != hipSuccess) break;
@@ -1330,6 +1351,20 @@ int kmi_lattice_autotune(kmi_lattice* L, int64_t steps_per_trial, double* best_m
         bb[0] = bx, bb[1] = by, bb[2] = nts, bb[3] = 0, bb[4] = 1;
       }
     }
+  }
+  // The lattice's own launch, on the shape found above, where no tile divides the extents and
+  // there is no other multi-step launch (get_temporal could not name it).
+  bool own = false, named = false;
+  for (int tile = 1; tile <= 14; ++tile) named = named || tb_eligible(L, tile);
+  if (L->Q == 19 && !named && e == hipSuccess) {
+    set_geometry(L, bb[0], bb[1], bb[2]);
+    L->tb_auto = true;
+    refresh_plan(L);
+    if (L->tb_tile) {
+      const double t = time_current();
+      if (e == hipSuccess && t < best) best = t, own = true;
+    }
+    L->tb_auto = false;
   }
   // Two- and three-step launches (the single-step shape found above serves remainders).
   const int zc_list[] = {1, 2, 3, 4, 6, 8, 12, 16};
@@ -1353,6 +1388,7 @@ int kmi_lattice_autotune(kmi_lattice* L, int64_t steps_per_trial, double* best_m
   set_geometry(L, bb[0], bb[1], bb[2]);
   L->tb_tile = bb[3];
   L->tb_zchunks = bb[4];
+  L->tb_auto = e == hipSuccess ? own : auto0;
   hipError_t e2 = hipMemcpyAsync(L->f[cur0], save_f, bytes, hipMemcpyDeviceToDevice, c->stream);
   if (e2 == hipSuccess && save_g)
     e2 = hipMemcpyAsync(L->g[cur0], save_g, gbytes, hipMemcpyDeviceToDevice, c->stream);

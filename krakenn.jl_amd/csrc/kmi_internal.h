@@ -52,6 +52,9 @@ int temporal_span(int tile);
 // bnd: a lattice with walls, moving walls, Zou–He faces or a solid mask (step2_tile_walled
 // tiles only; non-temporal stores whatever `nts` says).
 bool step2_tile_walled(int tile, int st);
+// Tile and z-split for a lattice whose user chose none (any x–y extent of at least a tile);
+// false: single steps are the faster ones.
+bool step2_plan(int st, bool bnd, const StepArgs& a, int& tile, int& zchunks);
 // Work-group → tile table of a walled multi-step launch (ring tiles first in each XCD band).
 void walled_tile_order(const StepArgs& a, int tile, int zchunks, std::vector<int>& order);
 hipError_t launch_step2(int st, int coll, int tile, int zchunks, bool nts, bool bnd, const StepArgs& a,

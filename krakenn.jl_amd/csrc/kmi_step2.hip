@@ -48,6 +48,10 @@ constexpr int group_index(int q) {
   return -1;
 }
 
+// First cell of tile t along an axis of n ≥ T cells.  Where T does not divide n the last tile
+// moves back to end at n − 1: the cells it shares with its neighbour are evaluated by both
+// groups from the same populations in the same order, and stored twice with the same bits.
+__host__ KMI_DEV int tile_start(int t, int T, int n) { return min(t * T, n - T); }
 KMI_DEV int wrap(int v, int n) { return v < 0 ? v + n : (v >= n ? v - n : v); }
 
 // Walled lattices: the kernels' template flag BND is 0 for a fully periodic lattice, 1 for
@@ -294,7 +298,7 @@ KMI_DEV void march2(const StepArgs& a, int zlen, int tx, int ty, int zc, typenam
 
   const int nx = a.nx, ny = a.ny, nz = a.nz;
   const long long P = a.plane;
-  const int x0 = tx * TX, y0 = ty * TY;
+  const int x0 = tb::tile_start(tx, TX, nx), y0 = tb::tile_start(ty, TY, ny);
   const int z0 = zc * zlen, z1 = min(z0 + zlen, nz);
   const E* __restrict__ fi = static_cast<const E*>(a.fi);
   E* __restrict__ fo = static_cast<E*>(a.fo);
@@ -424,7 +428,7 @@ KMI_DEV void march2_walled(const StepArgs& a, int zlen, int tx, int ty, int zc, 
 
   const int nx = a.nx, ny = a.ny, nz = a.nz;
   const long long P = a.plane;
-  const int x0 = tx * TX, y0 = ty * TY;
+  const int x0 = tb::tile_start(tx, TX, nx), y0 = tb::tile_start(ty, TY, ny);
   const int z0 = zc * zlen, z1 = min(z0 + zlen, nz);
   const E* __restrict__ fi = static_cast<const E*>(a.fi);
   E* __restrict__ fo = static_cast<E*>(a.fo);
@@ -636,7 +640,7 @@ KMI_DEV void march3(const StepArgs& a, int zlen, int tx, int ty, int zc, typenam
 
   const int nx = a.nx, ny = a.ny, nz = a.nz;
   const long long P = a.plane;
-  const int x0 = tx * TX, y0 = ty * TY;
+  const int x0 = tb::tile_start(tx, TX, nx), y0 = tb::tile_start(ty, TY, ny);
   const int z0 = zc * zlen, z1 = min(z0 + zlen, nz);
   const E* __restrict__ fi = static_cast<const E*>(a.fi);
   E* __restrict__ fo = static_cast<E*>(a.fo);
@@ -812,7 +816,7 @@ KMI_DEV void march3_walled(const StepArgs& a, int zlen, int tx, int ty, int zc, 
 
   const int nx = a.nx, ny = a.ny, nz = a.nz;
   const long long P = a.plane;
-  const int x0 = tx * TX, y0 = ty * TY;
+  const int x0 = tb::tile_start(tx, TX, nx), y0 = tb::tile_start(ty, TY, ny);
   const int z0 = zc * zlen, z1 = min(z0 + zlen, nz);
   const E* __restrict__ fi = static_cast<const E*>(a.fi);
   E* __restrict__ fo = static_cast<E*>(a.fo);
@@ -1050,8 +1054,8 @@ static void interior_tiles(bool per, int n, int T, int H, int ntiles, int& lo, i
   lo = 0;
   hi = ntiles;
   if (per) return;
-  while (lo < ntiles && lo * T - H < 1) ++lo;
-  while (hi > lo && (hi - 1) * T + T - 1 + H > n - 2) --hi;
+  while (lo < ntiles && tb::tile_start(lo, T, n) - H < 1) ++lo;
+  while (hi > lo && tb::tile_start(hi - 1, T, n) + T - 1 + H > n - 2) --hi;
   if (hi <= lo) lo = hi = 0;
 }
 
@@ -1064,12 +1068,67 @@ static bool lean_walls(const StepArgs& a) {
   return true;
 }
 
+// The multi-step launch of a lattice whose user chose none.  A group marches zlen planes and
+// the planes its lower and upper levels need beyond them (two steps 2, three steps 4);
+// `per_cu` groups share a CU, and once every CU is taken the groups run in rounds, so a launch
+// takes rounds · (zlen + 2·(span − 1)) · plane, and the pair (tile, z-split) with the least
+// time per step is taken.  `plane`: µs per marched plane with every CU taken, while the two
+// population buffers stay in the 256 MB last-level cache [0] and beyond it [1]; the model holds
+// within 6 % over cubes of 77³ to 256³, sides that the tile divides and others.  Against it
+// the single-step kernel at the rate it streams both buffers (5.4 TB/s in the cache; beyond it
+// 5.3 with rows of whole 128-byte lines, 4.5 otherwise).
+// Measured, single steps / the launch taken, µs per step:
+//   periodic  F64 96³ 43 / 31, 128³ 127 / 75, 150³ 231 / 126, 256³ 954 / 554; F32 128³ 64 / 36,
+//             150³ 132 / 67; F32S 107³ 32 / 19, 256³ 470 / 222; F16S 118³ 27 / 17, 256³ 240 / 181
+//   walled    F64 77³ 26.5 / 22.8, 128³ 129 / 91, 200³ 464 / 369; F32 128³ 66 / 41,
+//             200³ 241 / 174; F32S 96³ 23 / 19, 192³ 200 / 118
+bool step2_plan(int st, bool bnd, const StepArgs& a, int& tile, int& zchunks) {
+  struct Cand {
+    int tile, per_cu;
+    double plane[2];
+  };
+  static const Cand periodic[4][3] = {{{12, 1, {5.3, 7.8}}, {13, 1, {5.8, 7.9}}, {}},               // F64
+                                      {{11, 1, {4.7, 5.6}}, {9, 2, {4.6, 5.7}}, {12, 1, {3.5, 4.2}}},   // F32
+                                      {{11, 1, {3.8, 5.2}}, {9, 2, {3.6, 5.3}}, {12, 1, {2.7, 3.8}}},   // F32S
+                                      {{12, 2, {3.9, 5.2}}, {9, 2, {3.8, 4.1}}, {14, 3, {3.5, 4.8}}}};  // F16S
+  static const Cand walled[3][3] = {{{14, 1, {3.6, 4.8}}, {}, {}},                    // F64
+                                    {{12, 1, {3.6, 4.1}}, {14, 1, {2.6, 2.9}}, {}},   // F32
+                                    {{12, 1, {3.3, 3.8}}, {14, 1, {2.4, 2.8}}, {}}};  // F32S
+  tile = 0;
+  zchunks = 1;
+  const long long elem = st == KMI_STORE_F64 ? 8 : st == KMI_STORE_F16S ? 2 : 4;
+  // byte offsets within one population's plane are 32-bit in these kernels
+  if (a.plane * elem > (1LL << 32) || (bnd && (st == KMI_STORE_F16S || !lean_walls(a)))) return false;
+  const int kind = st == KMI_STORE_F64 ? 0 : st == KMI_STORE_F32 ? 1 : st == KMI_STORE_F32S ? 2 : 3;
+  const double bytes = 38.0 * elem * double(a.nx) * a.ny * a.nz;
+  const bool cached = bytes < 270e6;
+  double best = 0.95 * bytes / (cached ? 5.4e6 : a.nx * elem % 128 == 0 ? 5.3e6 : 4.5e6);
+  for (const Cand& c : bnd ? walled[kind] : periodic[kind]) {
+    int TX, TY;
+    if (!step2_tile(c.tile, st, TX, TY) || a.nx < TX || a.ny < TY) continue;
+    const long long columns = (long long)((a.nx + TX - 1) / TX) * ((a.ny + TY - 1) / TY);
+    const int span = temporal_span(c.tile);
+    for (int zc = 1; zc <= a.nz / 4; ++zc) {
+      const int zlen = (a.nz + zc - 1) / zc;
+      const long long groups = columns * ((a.nz + zlen - 1) / zlen);
+      const long long rounds = (groups + 256 * c.per_cu - 1) / (256 * c.per_cu);
+      const double t = double(rounds) * (zlen + 2 * (span - 1)) * c.plane[cached ? 0 : 1] / span;
+      if (t < best) {
+        best = t;
+        tile = c.tile;
+        zchunks = zc;
+      }
+    }
+  }
+  return tile != 0;
+}
+
 // One multi-step pass: every column tile × z-range in one launch, on the periodic kernel
 // (BND = 0) or, for a walled lattice, the walled one (BND = 2) with the interior block of
 // tiles (none when the lattice has a solid mask) marching on the interior variant.
 template <class Go>
 static hipError_t launch_tiles(bool bnd, int span, int TX, int TY, const StepArgs& a, int zchunks, Go&& go) {
-  const int ntx = a.nx / TX, nty = a.ny / TY;
+  const int ntx = (a.nx + TX - 1) / TX, nty = (a.ny + TY - 1) / TY;
   const int zlen = (a.nz + zchunks - 1) / zchunks;
   const int nzc = (a.nz + zlen - 1) / zlen;
   const int ntiles = ntx * nty * nzc;
@@ -1091,7 +1150,7 @@ void walled_tile_order(const StepArgs& a, int tile, int zchunks, std::vector<int
   order.clear();
   if (!step2_tile(tile, KMI_STORE_F32, TX, TY)) return;
   const int span = temporal_span(tile);
-  const int ntx = a.nx / TX, nty = a.ny / TY;
+  const int ntx = (a.nx + TX - 1) / TX, nty = (a.ny + TY - 1) / TY;
   const int zlen = (a.nz + zchunks - 1) / zchunks;
   const int ntiles = ntx * nty * ((a.nz + zlen - 1) / zlen);
   const int per_xcd = (ntiles + 7) / 8;

@@ -293,7 +293,9 @@ class Lattice:
         of the tile and its two-cell ring; FP64 only 7 and 9).  D2Q9 lattice without thermal populations, cut links or
         per-node faces: 1: 28×28 two steps, 2: 24×24 four (lattices of 160,000 cells and more
         without mask, forcing or thermal populations: strips marched in registers), 3: 56×8 four, 4: 16×16 eight,
-        5: 60×12 two, 6: 8×8 four, 7: 16×16 four, 8: 8×8 eight.  0: off.  Bit-identical to single steps."""
+        5: 60×12 two, 6: 8×8 four, 7: 16×16 four, 8: 8×8 eight.  0: off.  Bit-identical to single steps.
+        A D3Q19 lattice on which neither this nor set_launch nor autotune was called picks its own
+        multi-step launch where that is the faster one (`temporal` reports tile 0)."""
         self._chk(L.load().kmi_lattice_set_temporal(self._h, int(tile), int(zchunks)))
 
     @property
