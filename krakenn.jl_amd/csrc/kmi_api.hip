@@ -430,8 +430,9 @@ static bool tb_eligible(const kmi_lattice* L, int tile, bool any_extent = false)
   if (!L->bnd) return true;
   // walled lattices: halfway / moving-wall bounce-back, constant Zou–He faces and solid masks,
   // without forcing or cut links, on the walled tiles
-  if (!step2_tile_walled(tile, L->desc.storage) || L->desc.forcing != KMI_FORCE_NONE || !L->cut_cells.empty())
-    return false;
+  if (!step2_tile_walled(tile, L->desc.storage) || !L->cut_cells.empty()) return false;
+  // a constant body force: the lattice's own choice only
+  if (L->desc.forcing != KMI_FORCE_NONE && (!any_extent || L->desc.forcing == KMI_FORCE_GUO_FIELD)) return false;
   for (int f = 0; f < 6; ++f)
     if (L->desc.faces[f].kind > KMI_FACE_ZOUHE_PRESSURE) return false;
   return true;

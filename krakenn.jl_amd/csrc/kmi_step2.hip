@@ -175,12 +175,25 @@ struct Pops {
   }
 };
 
+// Collision of the walled two-step kernels under a constant body force (BGK only).
+constexpr int kCollGuo = 16;
+
 template <int ST, int COLL, class R>
 KMI_DEV void collide19(const R (&fp)[19], R (&fo)[19], const StepArgs& a) {
   constexpr bool SH = Store<ST>::shifted;
   if constexpr (ST == KMI_STORE_F16S) {
     if constexpr (COLL == KMI_TRT) collide_trt_shifted<19, true>(fp, fo, R(a.s_plus), R(a.s_minus));
     else collide_bgk_f16u<19>(fp, fo, R(a.omega));
+  } else if constexpr (COLL == kCollGuo) {
+    // the single-step kernel's operations: u = (Σcf + F/2)/ρ, then BGK with Guo's source
+    const R fx = R(a.fx), fy = R(a.fy), fz = R(a.fz);
+    const R m0 = zeroth_moment<19>(fp);
+    const R rho = SH ? R(1) + m0 : m0;
+    const R inv = R(1) / rho;
+    const R ux = (first_moment<19, 0>(fp) + fx / R(2)) * inv;
+    const R uy = (first_moment<19, 1>(fp) + fy / R(2)) * inv;
+    const R uz = (first_moment<19, 2>(fp) + fz / R(2)) * inv;
+    collide_guo19<SH>(fp, fo, m0, rho, ux, uy, uz, fx, fy, fz, R(a.omega));
   } else if constexpr (COLL == KMI_TRT) {
     collide_trt<19, SH>(fp, fo, R(a.s_plus), R(a.s_minus));
   } else {
@@ -1102,6 +1115,10 @@ bool step2_plan(int st, bool bnd, const StepArgs& a, int& tile, int& zchunks) {
   const int kind = st == KMI_STORE_F64 ? 0 : st == KMI_STORE_F32 ? 1 : st == KMI_STORE_F32S ? 2 : 3;
   const double bytes = 38.0 * elem * double(a.nx) * a.ny * a.nz;
   const bool cached = bytes < 270e6;
+  // a plane with Guo's source takes 1.34–1.45 times as long (F32 256×128×128 5.5 for 4.1 µs,
+  // F64 6.95 for 4.8): ducts F32 200×110×100 76.8 / 67.6 µs per step, 256×128×128 128 / 93,
+  // F64 256×128×128 245 / 230; single steps for what stays in the cache (150×75×61 21.6 / 25.7)
+  const double force = a.forcing ? 1.45 : 1.0;
   double best = 0.95 * bytes / (cached ? 5.4e6 : a.nx * elem % 128 == 0 ? 5.3e6 : 4.5e6);
   for (const Cand& c : bnd ? walled[kind] : periodic[kind]) {
     int TX, TY;
@@ -1112,7 +1129,7 @@ bool step2_plan(int st, bool bnd, const StepArgs& a, int& tile, int& zchunks) {
       const int zlen = (a.nz + zc - 1) / zc;
       const long long groups = columns * ((a.nz + zlen - 1) / zlen);
       const long long rounds = (groups + 256 * c.per_cu - 1) / (256 * c.per_cu);
-      const double t = double(rounds) * (zlen + 2 * (span - 1)) * c.plane[cached ? 0 : 1] / span;
+      const double t = double(rounds) * (zlen + 2 * (span - 1)) * force * c.plane[cached ? 0 : 1] / span;
       if (t < best) {
         best = t;
         tile = c.tile;
@@ -1266,8 +1283,32 @@ static hipError_t launch2_coll(int coll, int tile, bool nts, bool bnd, const Ste
                          : launch2_tile<ST, KMI_BGK>(tile, nts, bnd, a, zchunks, s);
 }
 
+// Constant body force (step2_plan's choices only): tiles 12 and 14 on the lean walled kernel.
+template <int ST>
+static hipError_t launch2_guo(int tile, const StepArgs& a, int zchunks, hipStream_t s) {
+  if (!lean_walls(a)) return hipErrorInvalidValue;
+  const auto go = [&](auto kernel, int nt) {
+    return [&a, s, kernel, nt](dim3 g, int zlen, int ntx, int nty, int ntiles, int per_xcd, int4 inner) -> hipError_t {
+      hipLaunchKernelGGL(kernel, g, dim3(unsigned(nt)), 0, s, a, zlen, ntx, nty, ntiles, per_xcd, inner);
+      return hipGetLastError();
+    };
+  };
+  if constexpr (ST != KMI_STORE_F64)
+    if (tile == 12) return launch_tiles(true, 2, 64, 8, a, zchunks, go((k_step2_d3q19<ST, kCollGuo, 64, 8, 704, true, 3>), 704));
+  if (tile == 14) return launch_tiles(true, 2, 32, 8, a, zchunks, go((k_step2_d3q19<ST, kCollGuo, 32, 8, 384, true, 3>), 384));
+  return hipErrorInvalidValue;
+}
+
 hipError_t launch_step2(int st, int coll, int tile, int zchunks, bool nts, bool bnd, const StepArgs& a,
                         hipStream_t s) {
+  if (a.forcing) {
+    switch (st) {
+      case KMI_STORE_F64: return launch2_guo<KMI_STORE_F64>(tile, a, zchunks, s);
+      case KMI_STORE_F32: return launch2_guo<KMI_STORE_F32>(tile, a, zchunks, s);
+      case KMI_STORE_F32S: return launch2_guo<KMI_STORE_F32S>(tile, a, zchunks, s);
+      default: return hipErrorInvalidValue;
+    }
+  }
   switch (st) {
     case KMI_STORE_F64: return launch2_coll<KMI_STORE_F64>(coll, tile, nts, bnd, a, zchunks, s);
     case KMI_STORE_F32: return launch2_coll<KMI_STORE_F32>(coll, tile, nts, bnd, a, zchunks, s);

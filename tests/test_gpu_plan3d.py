@@ -22,12 +22,38 @@ FACES = {
     "duct": dict(west=PERIODIC, east=PERIODIC, south=WALL, north=WALL, bottom=PERIODIC, top=PERIODIC),
     "couette": dict(west=PERIODIC, east=PERIODIC, south=PERIODIC, north=PERIODIC, bottom=WALL, top=LID),
 }
-SHAPES = [(128, 96, 101), (97, 105, 113), (129, 73, 131), (191, 95, 67), (66, 161, 127), (64, 200, 96)]
+SHAPES = [(128, 96, 101), (97, 105, 113), (129, 73, 131), (191, 95, 67), (66, 161, 127), (64, 200, 96),
+          (96, 39, 131), (187, 99, 96), (229, 81, 96), (159, 147, 40)]
 
 
 def _lattice(kmi, backend, faces, shape, storage, collision="trt"):
     return kmi.Lattice(kmi.make_desc("d3q19", *shape, 0.02, storage=storage, collision=collision,
                                      faces=FACES[faces]), backend)
+
+
+@pytest.mark.parametrize("storage", ["f64", "f32", "f32s"])
+@pytest.mark.parametrize("forcing", ["guo", "guo_plain"])
+def test_forced_default_launch_equals_single_steps(kmi, backend, storage, forcing):
+    """A constant body force in a duct, a moving-lid box and a fully periodic lattice."""
+    for k, (faces, shape) in enumerate([("duct", (96, 39, 131)), ("duct", (187, 135, 40)), ("duct", (124, 63, 96)),
+                                        ("ladd", (161, 129, 129)), ("periodic", (225, 119, 67)),
+                                        ("cavity", (96, 39, 131))]):
+        print(f"[plan] forced {faces} {storage} {shape}", flush=True)
+        d = kmi.make_desc("d3q19", *shape, 0.02, storage=storage, faces=FACES[faces], forcing=forcing,
+                          force=(2e-4, -1e-4, 3e-5))
+        got = []
+        for single in (False, True):
+            with kmi.Lattice(d, backend) as lat:
+                if single:
+                    lat.set_temporal(0)
+                else:
+                    with pytest.raises(kmi.KrakenError):
+                        lat.set_temporal(14, 1)
+                lat.init_equilibrium(*_fields(shape, k))
+                for n in (7, 33, 1):
+                    lat.step(n)
+                got.append(lat.download_raw())
+        assert np.array_equal(got[0], got[1]), (faces, storage, shape)
 
 
 def _fields(shape, seed):
