@@ -942,29 +942,57 @@ __global__ void k_epilogue(const float* __restrict__ P, int splits, long long MN
 // gradients): 256/SL outputs × SL split lanes per work-group, lane g summing splits g, g + SL,
 // …, the lane sums added in lane order (a fixed order: the result is deterministic).
 template <int SL>
-__global__ void __launch_bounds__(256) k_split_sum(const float* __restrict__ P, int splits, long long MN,
-                                                    float* __restrict__ out) {
+KMI_DEV void split_sum_group(float* part, int block, const float* __restrict__ P, int splits, long long MN,
+                             float* __restrict__ out) {
   constexpr int NO = 256 / SL;
-  __shared__ float part[SL][NO + 1];
   const int o = threadIdx.x % NO, g = threadIdx.x / NO;
-  const long long i = (long long)blockIdx.x * NO + o;
+  const long long i = (long long)block * NO + o;
   float z = 0.f;
   if (i < MN)
     for (int sp = g; sp < splits; sp += SL) z += P[(long long)sp * MN + i];
-  part[g][o] = z;
+  part[g * (NO + 1) + o] = z;
   __syncthreads();
   if (g == 0 && i < MN) {
     float t = 0.f;
-    for (int k = 0; k < SL; ++k) t += part[k][o];
+    for (int k = 0; k < SL; ++k) t += part[k * (NO + 1) + o];
     out[i] = t;
   }
 }
-static hipError_t launch_split_sum(const float* P, int splits, long long mn, float* out, hipStream_t s) {
-  if (splits > 256)
-    hipLaunchKernelGGL(k_split_sum<64>, dim3(unsigned((mn + 3) / 4)), dim3(256), 0, s, P, splits, mn, out);
-  else
-    hipLaunchKernelGGL(k_split_sum<16>, dim3(unsigned((mn + 15) / 16)), dim3(256), 0, s, P, splits, mn, out);
+// Up to three products per launch: the sums of the three convolutions' weight gradients took
+// 7.4 + 5.0 + 5.0 µs one after the other (32 samples of 128²), a few µs of work in a launch
+// that the next one waited for; together 11.7.
+struct SplitSums {
+  struct Job {
+    const float* P;
+    int splits, end;  // end: first work-group after this product's
+    long long mn;
+    float* out;
+  } job[3];
+  int n;
+};
+__global__ void __launch_bounds__(256) k_split_sum(const SplitSums c) {
+  __shared__ float part[64 * 5];
+  int k = 0;
+  while (k + 1 < c.n && int(blockIdx.x) >= c.job[k].end) ++k;
+  const SplitSums::Job& J = c.job[k];
+  const int block = int(blockIdx.x) - (k ? c.job[k - 1].end : 0);
+  if (J.splits > 256) split_sum_group<64>(part, block, J.P, J.splits, J.mn, J.out);
+  else split_sum_group<16>(part, block, J.P, J.splits, J.mn, J.out);
+}
+static void add_split_sum(SplitSums& c, const float* P, int splits, long long mn, float* out) {
+  const long long per = splits > 256 ? 4 : 16;
+  c.job[c.n] = {P, splits, (c.n ? c.job[c.n - 1].end : 0) + int((mn + per - 1) / per), mn, out};
+  ++c.n;
+}
+static hipError_t launch_split_sums(const SplitSums& c, hipStream_t s) {
+  if (!c.n) return hipSuccess;
+  hipLaunchKernelGGL(k_split_sum, dim3(unsigned(c.job[c.n - 1].end)), dim3(256), 0, s, c);
   return hipGetLastError();
+}
+static hipError_t launch_split_sum(const float* P, int splits, long long mn, float* out, hipStream_t s) {
+  SplitSums c{};
+  add_split_sum(c, P, splits, mn, out);
+  return launch_split_sums(c, s);
 }
 
 // Σ over `splits` partials, then dZ = Σ ⊙ SiLU'(Z) (or Σ); FP32 (when dZ is set) and BF16
@@ -992,29 +1020,45 @@ __global__ void __launch_bounds__(256) k_split_act(const float* __restrict__ P, 
   dZb[i] = f2bf(v);
 }
 
-// MSE loss partials and dY = 2 (Y − T) / count, stored in BF16 as [rows][Cp] (the padding
-// columns C … Cp − 1 are zero from allocation on).
+// MSE loss partials and dY = 2 (Y − T) / count, stored in BF16 as [rows][Cp], padding columns
+// C … Cp − 1 zero; image b's target is image idx[b] of T (b itself without idx).  A thread
+// takes whole rows (pixels), so a row of the gradient is one 16-byte store per 8 channels, and
+// the targets are read where the dataset keeps them: with one value per thread and a gathered
+// copy of the targets the two launches took 5.9 + 3.9 µs (32 samples of 128² × 3), now 7.1 in one.
 __global__ void __launch_bounds__(256) k_mse(const float* __restrict__ Y, const float* __restrict__ T,
-                                             long long n, int C, int Cp, uint16_t* __restrict__ dYb,
-                                             double* __restrict__ part) {
+                                             const int* __restrict__ idx, int rows, int image, int C, int Cp,
+                                             uint16_t* __restrict__ dYb, double* __restrict__ part) {
   __shared__ double lds[4];
   double acc = 0.0;
-  const float scale = 2.f / float(n);
-  for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-       i += (long long)gridDim.x * blockDim.x) {
-    const float d = Y[i] - T[i];
-    acc += double(d) * double(d);
-    const int ii = int(i), r = ii / C;  // element counts stay below 2^31 (kmi_nn_create)
-    dYb[(long long)r * Cp + (ii - r * C)] = f2bf(scale * d);
+  const float n = float((long long)rows * C), scale = 2.f / n;
+  for (unsigned r = blockIdx.x * blockDim.x + threadIdx.x; r < unsigned(rows); r += gridDim.x * blockDim.x) {
+    long long t = r;
+    if (idx) {
+      const unsigned b = r / unsigned(image);
+      t = (long long)idx[b] * image + (r - b * image);
+    }
+    const float* y = Y + (long long)r * C;
+    t *= C;
+    for (int c0 = 0; c0 < Cp; c0 += 8) {
+      uint32_t w[4];
+#pragma unroll
+      for (int k = 0; k < 8; ++k) {
+        float d = 0.f;
+        if (c0 + k < C) d = y[c0 + k] - T[t + c0 + k];
+        acc += double(d) * double(d);
+        const uint32_t h = f2bf(scale * d);
+        w[k / 2] = k % 2 ? w[k / 2] | h << 16 : h;
+      }
+      *reinterpret_cast<uint4*>(dYb + (long long)r * Cp + c0) = make_uint4(w[0], w[1], w[2], w[3]);
+    }
   }
   for (int off = 32; off > 0; off >>= 1) acc += __shfl_xor(acc, off, 64);
   if ((threadIdx.x & 63) == 0) lds[threadIdx.x >> 6] = acc;
   __syncthreads();
-  if (threadIdx.x == 0) part[blockIdx.x] = (lds[0] + lds[1] + lds[2] + lds[3]) / double(n);
+  if (threadIdx.x == 0) part[blockIdx.x] = (lds[0] + lds[1] + lds[2] + lds[3]) / double((long long)rows * C);
 }
 // One work-group: thread-strided sums in fixed order, then a fixed LDS tree.
-__global__ void __launch_bounds__(256) k_sum_parts(const double* __restrict__ part, int n, double* __restrict__ out) {
-  __shared__ double lds[256];
+KMI_DEV void sum_parts(double* lds, const double* __restrict__ part, int n, double* __restrict__ out) {
   const int t = threadIdx.x;
   double s = 0.0;
   for (int i = t; i < n; i += 256) s += part[i];
@@ -1025,6 +1069,10 @@ __global__ void __launch_bounds__(256) k_sum_parts(const double* __restrict__ pa
     __syncthreads();
   }
   if (t == 0) out[0] = lds[0];
+}
+__global__ void __launch_bounds__(256) k_sum_parts(const double* __restrict__ part, int n, double* __restrict__ out) {
+  __shared__ double lds[256];
+  sum_parts(lds, part, n, out);
 }
 
 __global__ void k_to_bf16(const float* __restrict__ x, long long n, uint16_t* __restrict__ y) {
@@ -1063,11 +1111,30 @@ __global__ void k_weight_copies(const WCopies c) {
   }
 }
 
-// Adam (β1 = 0.9, β2 = 0.999, ε = 1e-8) on the FP32 master weights; refreshes the BF16 copy.
-__global__ void k_adam(float* __restrict__ w, const float* __restrict__ g, float* __restrict__ m,
-                       float* __restrict__ v, uint16_t* __restrict__ wb, long long n, float lr,
-                       float c1, float c2) {
+// Adam (β1 = 0.9, β2 = 0.999, ε = 1e-8) on the FP32 master weights; refreshes the BF16 copy
+// and, for the convolutions, the copies in the direct kernels' layouts (their padding is zero
+// from kmi_nn_set_params on).  One more work-group sums the step's loss partials when there is
+// a slot for the sum.  Bound by the 30 bytes per weight (4.4 M weights 20 µs); as launches of
+// their own the copies took 4.2 µs and the sum 2.8.
+struct AdamCopies {
+  long long off[3];  // first weight of convolution k
+  int rows[3], co[3];
+  uint16_t* wt[3];   // [COP][rows] (null: none)
+  uint16_t* w3p;     // convolution 3 as [rows][Cp3] (null: none)
+  int Cp3;
+  const double* part;  // loss partials (slot null: no sum)
+  int nparts;
+  double* slot;
+};
+__global__ void __launch_bounds__(256) k_adam(float* __restrict__ w, const float* __restrict__ g, float* __restrict__ m,
+                                              float* __restrict__ v, uint16_t* __restrict__ wb, long long n, float lr,
+                                              float c1, float c2, const AdamCopies c) {
+  __shared__ double lds[256];
   const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (c.slot && blockIdx.x == gridDim.x - 1) {
+    sum_parts(lds, c.part, c.nparts, c.slot);
+    return;
+  }
   if (i >= n) return;
   const float gi = g[i];
   const float mi = 0.9f * m[i] + 0.1f * gi;
@@ -1076,19 +1143,24 @@ __global__ void k_adam(float* __restrict__ w, const float* __restrict__ g, float
   v[i] = vi;
   const float wi = w[i] - lr * (mi / c1) / (sqrtf(vi / c2) + 1e-8f);
   w[i] = wi;
-  wb[i] = f2bf(wi);
+  const uint16_t h = f2bf(wi);
+  wb[i] = h;
+  if (i < c.off[0]) return;
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    const long long e = i - c.off[k];
+    if (e < 0 || e >= (long long)c.rows[k] * c.co[k]) continue;
+    const int r = int(e) / c.co[k], o = int(e) - r * c.co[k];
+    if (c.wt[k]) c.wt[k][o * c.rows[k] + r] = h;
+    if (k == 2 && c.w3p) c.w3p[r * c.Cp3 + o] = h;
+  }
 }
 
-// Gather rows idx[0..B) of the device dataset into the batch buffers: grid (chunks, B), one
-// float4 of a target row per thread (a row holds (8·latent_hw)²·out_c floats, a multiple of
-// 4), and the first group of each row copies its input features.
-__global__ void k_gather(const float* __restrict__ X, const float* __restrict__ Y, const int* __restrict__ idx,
-                         int din, int dout4, float* __restrict__ xb, float* __restrict__ yb) {
-  const int b = blockIdx.y, src = idx[b], t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t < dout4)
-    reinterpret_cast<float4*>(yb)[(long long)b * dout4 + t] = reinterpret_cast<const float4*>(Y)[(long long)src * dout4 + t];
-  if (blockIdx.x == 0)
-    for (int i = threadIdx.x; i < din; i += blockDim.x) xb[(long long)b * din + i] = X[(long long)src * din + i];
+// Input features of the rows idx[0 … B) of the device dataset, in BF16.
+__global__ void k_gather(const float* __restrict__ X, const int* __restrict__ idx, int din, int n,
+                         uint16_t* __restrict__ xb) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) xb[i] = f2bf(X[(long long)idx[i / din] * din + i % din]);
 }
 
 static inline dim3 g1(long long n) { return dim3(unsigned((n + 255) / 256)); }
@@ -1358,9 +1430,11 @@ static hipError_t conv_dgrad(const Stage& S, int B, const uint16_t* dzb, const E
 
 // Weight and bias gradients of a stage into out = g + ow ([9 Ci][Co], then the Co biases):
 // chunks of input rows per work-group (about 256 work-groups, within P), partials summed in
-// chunk order.
+// chunk order by the launch that `sums` collects; they lie behind those it holds already, or
+// that launch is made first where P is too short for both.
 template <int CI, int HI>
-static hipError_t launch_wgrad(kmi_nn* N, const Stage& S, int B, const uint16_t* dzb, float* out, hipStream_t s) {
+static hipError_t launch_wgrad(kmi_nn* N, const Stage& S, int B, const uint16_t* dzb, float* out, SplitSums& sums,
+                               hipStream_t s) {
   const int nob = (S.Co + 15) / 16, steps = B * HI * HI / 128;
   const long long mn = (9LL * CI + 1) * S.Co;
   // about 1024 work-groups, with at most 8 MB of partials
@@ -1369,21 +1443,34 @@ static hipError_t launch_wgrad(kmi_nn* N, const Stage& S, int B, const uint16_t*
   nz = std::max<long long>(1, std::min<long long>(nz, (long long)N->P_elems / mn));
   const int spc = int((steps + nz - 1) / nz);
   nz = (steps + spc - 1) / spc;
+  float* P = N->P;
+  if (sums.n) {
+    const SplitSums::Job& last = sums.job[sums.n - 1];
+    P = const_cast<float*>(last.P) + last.splits * last.mn;
+    if (P + nz * mn > N->P + N->P_elems) {
+      if (hipError_t e = launch_split_sums(sums, s); e != hipSuccess) return e;
+      sums.n = 0;
+      P = N->P;
+    }
+  }
   hipLaunchKernelGGL((k_conv_wgrad<CI, HI>), dim3(unsigned(nz), unsigned(nob)), dim3(64 * (CI / 16)), 0, s, S.in, dzb,
-                     S.Cp, S.Co, steps, spc, N->P);
+                     S.Cp, S.Co, steps, spc, P);
   if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
-  return launch_split_sum(N->P, int(nz), mn, out, s);
+  add_split_sum(sums, P, int(nz), mn, out);
+  return hipSuccess;
 }
 template <int CI>
-static hipError_t conv_wgrad_ci(kmi_nn* N, const Stage& S, int B, const uint16_t* dzb, float* out, hipStream_t s) {
+static hipError_t conv_wgrad_ci(kmi_nn* N, const Stage& S, int B, const uint16_t* dzb, float* out, SplitSums& sums,
+                                hipStream_t s) {
   switch (S.Hi) {
-    case 16: return launch_wgrad<CI, 16>(N, S, B, dzb, out, s);
-    case 32: return launch_wgrad<CI, 32>(N, S, B, dzb, out, s);
-    default: return launch_wgrad<CI, 64>(N, S, B, dzb, out, s);
+    case 16: return launch_wgrad<CI, 16>(N, S, B, dzb, out, sums, s);
+    case 32: return launch_wgrad<CI, 32>(N, S, B, dzb, out, sums, s);
+    default: return launch_wgrad<CI, 64>(N, S, B, dzb, out, sums, s);
   }
 }
-static hipError_t conv_wgrad(kmi_nn* N, const Stage& S, int B, const uint16_t* dzb, float* out, hipStream_t s) {
-  return S.Ci == 64 ? conv_wgrad_ci<64>(N, S, B, dzb, out, s) : conv_wgrad_ci<32>(N, S, B, dzb, out, s);
+static hipError_t conv_wgrad(kmi_nn* N, const Stage& S, int B, const uint16_t* dzb, float* out, SplitSums& sums,
+                             hipStream_t s) {
+  return S.Ci == 64 ? conv_wgrad_ci<64>(N, S, B, dzb, out, sums, s) : conv_wgrad_ci<32>(N, S, B, dzb, out, sums, s);
 }
 
 static void stages(const kmi_nn* N, Stage (&st)[3]) {
@@ -1393,13 +1480,14 @@ static void stages(const kmi_nn* N, Stage (&st)[3]) {
   st[2] = {N->h4b, N->H2, d.c2, d.out_c, N->Cp3, w3_bf16(N), N->oC3, N->obc3};
 }
 
-// Forward pass for batch B from N->x (FP32) into N->y.
-static int nn_forward(kmi_nn* N, int B) {
+// Forward pass for batch B from N->x (FP32), or from N->xb where that is filled, into N->y.
+static int nn_forward(kmi_nn* N, int B, bool have_xb = false) {
   const kmi_nn_desc& d = N->d;
   hipStream_t s = N->ctx->stream;
   const uint16_t* wb = N->wb;
   const float* w = N->w;
-  hipLaunchKernelGGL(k_to_bf16, g1((long long)B * d.in_dim), dim3(256), 0, s, N->x, (long long)B * d.in_dim, N->xb);
+  if (!have_xb)
+    hipLaunchKernelGGL(k_to_bf16, g1((long long)B * d.in_dim), dim3(256), 0, s, N->x, (long long)B * d.in_dim, N->xb);
   // dense 1: [B, in] · W1[in, hidden], bias, SiLU
   NN_CHECK((mm<64, 64, 2>(B, d.hidden, d.in_dim, 1, DenseK{N->xb, d.in_dim, B, d.in_dim},
                           DenseR{wb + N->oW1, d.hidden, d.hidden, d.in_dim},
@@ -1438,6 +1526,12 @@ static int nn_backward(kmi_nn* N, int B) {
   // gradient w.r.t. the stage output pre-activation in BF16 [M, Cp]
   const uint16_t* dzb = N->dyb;
   int pp = 0;
+  SplitSums sums{};  // weight-gradient partials in P that wait for their sum
+  const auto finish_sums = [&]() -> hipError_t {
+    const hipError_t e = launch_split_sums(sums, s);
+    sums.n = 0;
+    return e;
+  };
   for (int k = 2; k >= 0; --k) {
     const Stage& S = st[k];
     const int Ho = 2 * S.Hi, Mo = B * Ho * Ho;
@@ -1445,8 +1539,9 @@ static int nn_backward(kmi_nn* N, int B) {
     // of ones below A: its result row is the bias gradient Σ_pixels dZ[pixel, o], which the
     // flat layout stores right after the weights (g + ob = g + ow + 9 Ci Co)
     if (wgrad_direct(S.Ci, S.Hi)) {
-      NN_CHECK(conv_wgrad(N, S, B, dzb, g + S.ow, s));
+      NN_CHECK(conv_wgrad(N, S, B, dzb, g + S.ow, sums, s));
     } else {
+      NN_CHECK(finish_sums());
       const int Mw = 9 * S.Ci + 1;
       const int sp = pick_splits(N, 64, S.Co > 32 ? 64 : (S.Co > 16 ? 32 : 16), Mw, S.Co, Mo, 2048, 512);
       NN_CHECK(mm_wgrad(Mw, S.Co, Mo, sp, WithOnes<ConvWgradA>{ConvWgradA{S.in, B, S.Hi, S.Ci}, 9 * S.Ci, Mo},
@@ -1465,6 +1560,7 @@ static int nn_backward(kmi_nn* N, int B) {
       NN_CHECK(mm_by_n(Mi, S.Ci, Kd, 1, ConvDgradA{dzb, B, S.Hi, S.Cp}, ConvDgradB{S.wbf, S.Ci, S.Cp},
                        EpiActGrad{zin[k], nullptr, N->dzb[pp], 1}, s));
     } else {
+      NN_CHECK(finish_sums());
       NN_CHECK(mm_by_n(Mi, S.Ci, Kd, spd, ConvDgradA{dzb, B, S.Hi, S.Cp}, ConvDgradB{S.wbf, S.Ci, S.Cp},
                        EpiStore{N->P}, s));
       int sp2 = 1;
@@ -1477,6 +1573,7 @@ static int nn_backward(kmi_nn* N, int B) {
     dzb = N->dzb[pp];
     pp ^= 1;
   }
+  NN_CHECK(finish_sums());
   // dense 2: dZ2 is in dzb as [B, L]; weight and bias gradients (a row of ones below
   // h1ᵀ; b2 follows W2 in the flat layout)
   NN_CHECK((mm<64, 64, 2>(d.hidden + 1, N->L, B, 1,
@@ -1502,31 +1599,29 @@ static int nn_backward(kmi_nn* N, int B) {
   return KMI_OK;
 }
 
-// MSE loss and its gradient dY; the loss lands in `slot` (device; default lout) and, when
-// `loss` is given, is read back.
-static int nn_loss(kmi_nn* N, int B, double* loss, double* slot = nullptr) {
-  hipStream_t s = N->ctx->stream;
+// MSE loss partials (`nb` of them, in lpart) and the loss gradient dY against `target`, image b
+// of it at idx[b] (b without idx).
+static int nn_loss(kmi_nn* N, int B, const float* target, const int* idx, int* nb) {
   const long long n = out_elems(N, B);
-  const int nb = int(std::min<long long>(1024, (n + 255) / 256));
-  if (!slot) slot = N->lout;
-  hipLaunchKernelGGL(k_mse, dim3(unsigned(nb)), dim3(256), 0, s, N->y, N->tgt, n, N->d.out_c, N->Cp3, N->dyb,
-                     N->lpart);
-  hipLaunchKernelGGL(k_sum_parts, dim3(1), dim3(256), 0, s, N->lpart, nb, slot);
+  *nb = int(std::min<long long>(1024, (n + 255) / 256));
+  hipLaunchKernelGGL(k_mse, dim3(unsigned(*nb)), dim3(256), 0, N->ctx->stream, N->y, target, idx,
+                     B * N->H3 * N->H3, N->H3 * N->H3, N->d.out_c, N->Cp3, N->dyb, N->lpart);
   NN_CHECK(hipGetLastError());
-  if (loss) {
-    NN_CHECK(hipMemcpyAsync(loss, slot, 8, hipMemcpyDeviceToHost, s));
-    NN_CHECK(hipStreamSynchronize(s));
-  }
   return KMI_OK;
 }
 
-static int nn_adam(kmi_nn* N, float lr) {
+// One Adam step; with `slot` (device) the `nb` loss partials are summed into it.
+static int nn_adam(kmi_nn* N, float lr, int nb = 0, double* slot = nullptr) {
   N->adam_t += 1;
+  const kmi_nn_desc& d = N->d;
   const float c1 = 1.f - powf(0.9f, float(N->adam_t)), c2 = 1.f - powf(0.999f, float(N->adam_t));
-  hipLaunchKernelGGL(k_adam, g1(N->nparam), dim3(256), 0, N->ctx->stream, N->w, N->g, N->m, N->v, N->wb, N->nparam,
-                     lr, c1, c2);
+  AdamCopies c{{N->oC1, N->oC2, N->oC3}, {9 * d.latent_c, 9 * d.c1, 9 * d.c2}, {d.c1, d.c2, d.out_c},
+               {N->wt[0], N->wt[1], N->wt[2]}, N->w3p, N->Cp3, N->lpart, nb, slot};
+  dim3 grid = g1(N->nparam);
+  if (slot) grid.x += 1;
+  hipLaunchKernelGGL(k_adam, grid, dim3(256), 0, N->ctx->stream, N->w, N->g, N->m, N->v, N->wb, N->nparam, lr, c1, c2,
+                     c);
   NN_CHECK(hipGetLastError());
-  NN_CHECK(refresh_weight_copies(N, N->ctx->stream));
   return KMI_OK;
 }
 
@@ -1673,7 +1768,14 @@ int kmi_nn_loss_grad(kmi_nn* N, int32_t B, const float* x, const float* target, 
   const HostSeg in{const_cast<float*>(target), N->tgt, size_t(out_elems(N, B)) * 4};
   KMI_HIP(c, copy_to_device(c, &in, 1));
   if (int rc = nn_forward(N, B)) return rc;
-  if (int rc = nn_loss(N, B, loss)) return rc;
+  int nb = 0;
+  if (int rc = nn_loss(N, B, N->tgt, nullptr, &nb)) return rc;
+  if (loss) {
+    hipLaunchKernelGGL(k_sum_parts, dim3(1), dim3(256), 0, c->stream, N->lpart, nb, N->lout);
+    KMI_HIP(c, hipGetLastError());
+    KMI_HIP(c, hipMemcpyAsync(loss, N->lout, 8, hipMemcpyDeviceToHost, c->stream));
+    KMI_HIP(c, hipStreamSynchronize(c->stream));
+  }
   if (int rc = nn_backward(N, B)) return rc;
   if (grad) {
     const HostSeg out{grad, N->g, size_t(N->nparam) * 4};
@@ -1725,7 +1827,6 @@ int kmi_nn_train_epochs(kmi_nn* N, int32_t epochs, int32_t B, float lr, uint64_t
   if (int rc = nn_batch_ok(N, B)) return rc;
   if (B > N->dsN) return fail(c, KMI_ERR_ARG, "kmi_nn_train_epochs: batch larger than the dataset");
   KMI_HIP(c, hipSetDevice(c->device));
-  const long long dout = out_elems(N, 1);
   std::vector<int> perm(N->dsN);
   uint64_t s = seed;
   const int nb = N->dsN / B;
@@ -1736,13 +1837,15 @@ int kmi_nn_train_epochs(kmi_nn* N, int32_t epochs, int32_t B, float lr, uint64_t
     KMI_HIP(c, hipStreamSynchronize(c->stream));
     KMI_HIP(c, hipMemcpyAsync(N->perm_d, perm.data(), (size_t)N->dsN * 4, hipMemcpyHostToDevice, c->stream));
     for (int b = 0; b < nb; ++b) {
-      hipLaunchKernelGGL(k_gather, dim3(unsigned((dout / 4 + 255) / 256), unsigned(B)), dim3(256), 0, c->stream,
-                         N->dsX, N->dsY, N->perm_d + (size_t)b * B, N->d.in_dim, int(dout / 4), N->x, N->tgt);
+      const int* idx = N->perm_d + (size_t)b * B;
+      hipLaunchKernelGGL(k_gather, g1((long long)B * N->d.in_dim), dim3(256), 0, c->stream, N->dsX, idx, N->d.in_dim,
+                         B * N->d.in_dim, N->xb);
       KMI_HIP(c, hipGetLastError());
-      if (int rc = nn_forward(N, B)) return rc;
-      if (int rc = nn_loss(N, B, nullptr, N->lhist + b)) return rc;
+      int parts = 0;
+      if (int rc = nn_forward(N, B, true)) return rc;
+      if (int rc = nn_loss(N, B, N->dsY, idx, &parts)) return rc;
       if (int rc = nn_backward(N, B)) return rc;
-      if (int rc = nn_adam(N, lr)) return rc;
+      if (int rc = nn_adam(N, lr, parts, N->lhist + b)) return rc;
     }
   }
   std::vector<double> lh(nb);
