@@ -5,9 +5,19 @@
 // the release of the written lines), 3–6 µs.  This kernel pays that cost once per K steps.
 // A work-group loads its TW × TH tile plus a K-cell ring of the t populations into LDS,
 // advances the whole region K steps in place (each step needs one cell less on every side),
-// and writes the tile's t+K populations.  One work-item per cell of the region (1024), so
-// each in-LDS step is one dependent chain per work-item with 16 waves per CU to hide it;
-// the cost is the ring's re-evaluation.
+// and writes the tile's t+K populations.  One work-item per cell of the region, so each in-LDS
+// step is one dependent chain per work-item with up to 16 waves per CU to hide it; the cost is
+// the ring's re-evaluation.
+//
+// Step s needs the (EW − 2s) × (EH − 2s) cells inside the region.  In FP64 they are dealt to the
+// work-items afresh at every step, consecutive cells to consecutive lanes, so the waves that a
+// step needs shrink with it: 8, 7, 6, 4, 4, 3, 2, 1 of the 9 waves of the 8×8 tile with 8 steps,
+// against 9, 9, 7, 7, 7, 5, 5, 3 with active lanes, up to three on a SIMD, when every cell keeps
+// its work-item (128² BGK cavity, µs per step: 2.17 kept, 1.96 dealt; 256² on 16×16 tiles with 4
+// steps 3.49 and 3.30).  In FP32 the chain of one wave sets the time, and a kept cell's indices
+// and wall tests stay out of the step loop: 128² F32S cavity 1.56 kept and 1.72 dealt, 512×256
+// F32S Rayleigh–Bénard 4.19 and 4.63.  The second launch bound keeps 4 waves per SIMD (FP64 BGK
+// 130 VGPRs without it: 256² on 8×8 tiles with 4 steps 4.37 instead of 3.72).
 //
 // Scope: D2Q9 BGK / TRT / MRT with periodic, wall, moving-wall and constant Zou–He
 // (velocity or pressure) faces, bounce-back or inert masks and Guo forcing (constant or
@@ -22,15 +32,15 @@
 namespace kmi {
 
 template <int ST, int COLL, int TW, int TH, int K, bool THM>
-__global__ void __launch_bounds__((TW + 2 * K) * (TH + 2 * K)) k_step_tb2d(const StepArgs a) {
+__global__ void __launch_bounds__((TW + 2 * K) * (TH + 2 * K), 4) k_step_tb2d(const StepArgs a) {
   using S = Store<ST>;
   using E = typename S::elem;
   using R = typename S::real;
   using GS = Store<thermal_storage(ST)>;
   using GE = typename GS::elem;
   constexpr bool SH = S::shifted;
-  constexpr int EW = TW + 2 * K, EH = TH + 2 * K, NE = EW * EH, NT = NE;
-  constexpr int EPT = 1;
+  constexpr int EW = TW + 2 * K, EH = TH + 2 * K, NE = EW * EH;
+  constexpr bool DEAL = sizeof(R) == 8;
   __shared__ R L[(THM ? 18 : 9) * NE];
   R* const G = L + 9 * NE;  // thermal populations (THM)
   const GE* __restrict__ gi = static_cast<const GE*>(a.gi);
@@ -49,26 +59,35 @@ __global__ void __launch_bounds__((TW + 2 * K) * (TH + 2 * K)) k_step_tb2d(const
     return (perx || (ux >= 0 && ux < nx)) && (pery || (uy >= 0 && uy < ny));
   };
 
-  for (int e = tid; e < NE; e += NT) {
-    const int ux = ox + e % EW, uy = oy + e / EW;
-    if (!inside(ux, uy)) continue;
+  if (const int ux = ox + tid % EW, uy = oy + tid / EW; inside(ux, uy)) {
     const long long self = wx(ux) + (long long)nx * wy(uy);
     sfor<9>([&](auto qc) {
       constexpr int q = decltype(qc)::value;
-      L[q * NE + e] = S::ld(fi, self + q * P);
-      if constexpr (THM) G[q * NE + e] = GS::ld(gi, self + q * P);
+      L[q * NE + tid] = S::ld(fi, self + q * P);
+      if constexpr (THM) G[q * NE + tid] = GS::ld(gi, self + q * P);
     });
   }
   __syncthreads();
 
-  R nv[EPT][9], gv[EPT][9];
+  R nv[9], gv[9];
   for (int s = 1; s <= K; ++s) {
-#pragma unroll
-    for (int r = 0; r < EPT; ++r) {
-      const int e = tid + r * NT;
-      const int ex = e % EW, ey = e / EW;
-      const int ux = ox + ex, uy = oy + ey;
-      if (e >= NE || ex < s || ex >= EW - s || ey < s || ey >= EH - s || !inside(ux, uy)) continue;
+    int ex = tid % EW, ey = tid / EW;
+    if constexpr (DEAL) {
+      // cell tid of the step's (EW − 2s) × (EH − 2s) cells; ⌊tid / w⌋ = tid·⌈2^16/w⌉ >> 16 for
+      // tid < 1024 and w ≤ 64 (tid·(w − 1) < 2^16)
+      const int w = EW - 2 * s;
+      unsigned m = 0;
+      sfor<K>([&](auto kc) {
+        constexpr int k = decltype(kc)::value + 1, wk = EW - 2 * k;
+        if (s == k) m = (65536 + wk - 1) / wk;
+      });
+      const int row = int(unsigned(tid) * m >> 16);
+      ex = s + tid - row * w;
+      ey = s + row;
+    }
+    const int e = ex + ey * EW, ux = ox + ex, uy = oy + ey;
+    const bool active = (DEAL || (ex >= s && ex < EW - s && ey >= s)) && ey < EH - s && inside(ux, uy);
+    if (active) {
       const int i = wx(ux), j = wy(uy);
       const long long self = i + (long long)nx * j;
       // a link whose source lies beyond a non-periodic face bounces back (k_step's rule)
@@ -140,7 +159,7 @@ __global__ void __launch_bounds__((TW + 2 * K) * (TH + 2 * K)) k_step_tb2d(const
         } else {
           collide_guo<SH>(fp, fr, m0, rho, uxf, uyf, fx, fy, R(a.omega));
         }
-        sfor<9>([&](auto qc) { gv[r][decltype(qc)::value] = gr[decltype(qc)::value]; });
+        sfor<9>([&](auto qc) { gv[decltype(qc)::value] = gr[decltype(qc)::value]; });
       } else if (solid && a.solid_inert) {
         sfor<9>([&](auto qc) { fr[decltype(qc)::value] = SH ? R(0) : R(Lat<9>::w[decltype(qc)::value]); });
       } else if (solid) {
@@ -165,39 +184,29 @@ __global__ void __launch_bounds__((TW + 2 * K) * (TH + 2 * K)) k_step_tb2d(const
       }
       sfor<9>([&](auto qc) {
         constexpr int q = decltype(qc)::value;
-        nv[r][q] = fr[q];
+        nv[q] = fr[q];
       });
     }
-    if (s == K) break;
+    if (s == K) {
+      // the tile's own cells: step t+K straight from registers
+      if (active && ux < nx && uy < ny) {
+        const long long self = ux + (long long)nx * uy;
+        sfor<9>([&](auto qc) {
+          constexpr int q = decltype(qc)::value;
+          S::template st<false>(fo, self + q * P, nv[q]);
+          if constexpr (THM) GS::template st<false>(go, self + q * P, gv[q]);
+        });
+      }
+      break;
+    }
     __syncthreads();  // every step-s read of L is done
-#pragma unroll
-    for (int r = 0; r < EPT; ++r) {
-      const int e = tid + r * NT;
-      const int ex = e % EW, ey = e / EW;
-      if (e >= NE || ex < s || ex >= EW - s || ey < s || ey >= EH - s || !inside(ox + ex, oy + ey)) continue;
+    if (active)
       sfor<9>([&](auto qc) {
         constexpr int q = decltype(qc)::value;
-        L[q * NE + e] = storage_round<ST>(nv[r][q]);
-        if constexpr (THM) G[q * NE + e] = storage_round<thermal_storage(ST)>(gv[r][q]);
+        L[q * NE + e] = storage_round<ST>(nv[q]);
+        if constexpr (THM) G[q * NE + e] = storage_round<thermal_storage(ST)>(gv[q]);
       });
-    }
     __syncthreads();
-  }
-
-  // the tile's own cells: step t+K straight from registers
-#pragma unroll
-  for (int r = 0; r < EPT; ++r) {
-    const int e = tid + r * NT;
-    const int ex = e % EW, ey = e / EW;
-    if (e >= NE || ex < K || ex >= K + TW || ey < K || ey >= K + TH) continue;
-    const int ux = ox + ex, uy = oy + ey;
-    if (ux >= nx || uy >= ny) continue;
-    const long long self = ux + (long long)nx * uy;
-    sfor<9>([&](auto qc) {
-      constexpr int q = decltype(qc)::value;
-      S::template st<false>(fo, self + q * P, nv[r][q]);
-      if constexpr (THM) GS::template st<false>(go, self + q * P, gv[r][q]);
-    });
   }
 }
 
