@@ -31,8 +31,16 @@
 
 namespace kmi {
 
+// Whether a step writes a second buffer instead of the one it reads, which saves one of its two
+// barriers: the 8×8 tile with 8 steps (83 KB in FP64, one group per CU, as many as its lattices
+// have), 128² BGK cavity F64 1.96 → 1.89, F32S 1.56 → 1.52 µs per step.  The other tiles also
+// serve lattices with several groups per CU, which lose more by the LDS (330² F32 on 16×16
+// tiles with 4 steps 3.9 → 4.5).
+constexpr bool tb2d_two_buffers(int TW, int TH, int K, bool thm) { return !thm && K == 8 && TW == 8 && TH == 8; }
+
 template <int ST, int COLL, int TW, int TH, int K, bool THM>
-__global__ void __launch_bounds__((TW + 2 * K) * (TH + 2 * K), 4) k_step_tb2d(const StepArgs a) {
+__global__ void __launch_bounds__((TW + 2 * K) * (TH + 2 * K), tb2d_two_buffers(TW, TH, K, THM) ? 3 : 4)
+    k_step_tb2d(const StepArgs a) {
   using S = Store<ST>;
   using E = typename S::elem;
   using R = typename S::real;
@@ -41,8 +49,11 @@ __global__ void __launch_bounds__((TW + 2 * K) * (TH + 2 * K), 4) k_step_tb2d(co
   constexpr bool SH = S::shifted;
   constexpr int EW = TW + 2 * K, EH = TH + 2 * K, NE = EW * EH;
   constexpr bool DEAL = sizeof(R) == 8;
-  __shared__ R L[(THM ? 18 : 9) * NE];
-  R* const G = L + 9 * NE;  // thermal populations (THM)
+  constexpr bool TWOBUF = tb2d_two_buffers(TW, TH, K, THM);
+  constexpr int NV = (THM ? 18 : 9) * NE;
+  __shared__ R lds[(TWOBUF ? 2 : 1) * NV];
+  R* L = lds;
+  R* G = L + 9 * NE;  // thermal populations (THM)
   const GE* __restrict__ gi = static_cast<const GE*>(a.gi);
   GE* __restrict__ go = static_cast<GE*>(a.go);
   const int nx = a.nx, ny = a.ny;
@@ -199,7 +210,12 @@ __global__ void __launch_bounds__((TW + 2 * K) * (TH + 2 * K), 4) k_step_tb2d(co
       }
       break;
     }
-    __syncthreads();  // every step-s read of L is done
+    if constexpr (TWOBUF) {
+      L = lds + (s & 1) * NV;
+      G = L + 9 * NE;
+    } else {
+      __syncthreads();  // every step-s read of L is done
+    }
     if (active)
       sfor<9>([&](auto qc) {
         constexpr int q = decltype(qc)::value;
