@@ -79,3 +79,23 @@ def test_reductions_repeat(kmi, backend):
             # compensated sum of FP64 values: a few ulps of the exact one
             assert abs(first[0] - math.fsum(m["rho"].ravel())) <= 4e-16 * first[0]
             assert first[3] == pytest.approx(float(np.max(np.hypot(m["ux"], m["uy"]))), rel=1e-15)
+
+
+@pytest.mark.parametrize("cells", [256, 257, 513, 2304, 3841, 4096, 4097])
+def test_reductions_of_few_groups(kmi, backend, cells):
+    """One group, two to sixteen (summed by the last of them) and seventeen."""
+    import math
+
+    r = np.random.default_rng(cells)
+    shape = (cells, 1) if cells % 2 else (cells // 2, 2)
+    with kmi.Lattice(kmi.make_desc("d2q9", *shape, 1, 0.05), backend) as lat:
+        lat.init_equilibrium(1 + 0.1 * r.uniform(-1, 1, shape), 0.02 * r.uniform(-1, 1, shape),
+                             0.02 * r.uniform(-1, 1, shape))
+        mass, mom, speed = lat.reduce("mass"), lat.reduce("momentum"), lat.reduce("max_speed")
+        m = lat.moments()
+        # compensated sums of FP64 values: a few ulps of the exact ones (of Σ|x| for the momentum)
+        assert abs(mass - math.fsum(m["rho"].ravel())) <= 4e-16 * mass
+        for k, u in enumerate(("ux", "uy")):
+            x = (m["rho"] * m[u]).ravel()
+            assert abs(mom[k] - math.fsum(x)) <= 4e-16 * np.abs(x).sum() + 1e-300
+        assert speed == pytest.approx(float(np.max(np.hypot(m["ux"], m["uy"]))), rel=1e-15)
