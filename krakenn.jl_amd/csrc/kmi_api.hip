@@ -330,6 +330,7 @@ static void build_args(kmi_lattice* L) {
   a.coupling = d.coupling;
   a.forcing = d.forcing != KMI_FORCE_NONE;
   a.solid_inert = d.solid_mode == KMI_SOLID_INERT;
+  a.mask = L->mask;
   a.cut_slot = L->cut_slot;
   a.cut_rec = L->cut_rec;
   a.fx = d.force[0];
@@ -407,9 +408,10 @@ static void default_geometry(kmi_lattice* L) {
 }
 
 // Whether multi-step launches with `tile` apply.  D3Q19: BGK/TRT without thermal populations,
-// the x–y extent a multiple of the tile and at least 4 planes in z; fully periodic lattices
-// without mask on any tile, walled ones (walls, moving walls, constant Zou–He faces, solid
-// mask; no forcing, no cut links) on the walled tiles (12, 14; 9 except FP64; not F16S).  D2Q9 (k_step_tb2d):
+// the x–y extent a multiple of the tile (any_extent: at least the tile) and at least 4 planes in
+// z; fully periodic lattices without mask on any tile, walled ones (walls, moving walls, constant
+// Zou–He faces, solid mask; no cut links) on the walled tiles (12, 14; 9 except FP64; not F16S),
+// under a constant body force only with any_extent and without mask.  D2Q9 (k_step_tb2d):
 // no cut links, faces periodic / wall / moving wall / constant Zou–He only (thermal lattices
 // included), and a lattice of at least the tile plus its ring on each axis.
 static bool tb_eligible(const kmi_lattice* L, int tile, bool any_extent = false) {
@@ -429,10 +431,11 @@ static bool tb_eligible(const kmi_lattice* L, int tile, bool any_extent = false)
   if (!any_extent && (L->desc.nx % TX != 0 || L->desc.ny % TY != 0)) return false;
   if (!L->bnd) return true;
   // walled lattices: halfway / moving-wall bounce-back, constant Zou–He faces and solid masks,
-  // without forcing or cut links, on the walled tiles
+  // without cut links, on the walled tiles
   if (!step2_tile_walled(tile, L->desc.storage) || !L->cut_cells.empty()) return false;
-  // a constant body force: the lattice's own choice only
-  if (L->desc.forcing != KMI_FORCE_NONE && (!any_extent || L->desc.forcing == KMI_FORCE_GUO_FIELD)) return false;
+  // a constant body force: the lattice's own choice only, on the kernel without a mask
+  if (L->desc.forcing != KMI_FORCE_NONE && (!any_extent || L->mask || L->desc.forcing == KMI_FORCE_GUO_FIELD))
+    return false;
   for (int f = 0; f < 6; ++f)
     if (L->desc.faces[f].kind > KMI_FACE_ZOUHE_PRESSURE) return false;
   return true;
@@ -471,7 +474,6 @@ static int launch_one(kmi_lattice* L, hipStream_t s, bool multi = false) {
   a.fo = L->f[L->cur ^ 1];
   a.gi = L->g[L->cur];
   a.go = L->g[L->cur ^ 1];
-  a.mask = L->mask;
   // the table only for the tile and z-split it was built for (any other launch keeps the
   // default order, which covers every tile as well)
   a.tile_order = multi && L->bnd && L->Q == 19 && !L->tb_auto && L->order && L->order_key[0] == L->tb_tile &&
