@@ -31,15 +31,36 @@
 
 namespace kmi {
 
+// LATE: the tile's own cells are stored after the step loop instead of in its last step, which
+// takes 14–32 VGPRs less.  A launch whose groups spread over the CUs gains by the stores in the
+// loop (2–5 %); where groups share a CU the registers decide how many do.
+//   - regions of 576 cells (9 waves a group) from 257 groups on: FP32 70 VGPRs instead of 84, three
+//     groups a CU instead of one or two: 900×300 BGK cavity on 16×16 tiles 5.98 instead of 8.36 µs a
+//     step, on 8×8 tiles with 8 steps 14.2 instead of 19.5; thermal 90 VGPRs instead of 120, 900×300
+//     Rayleigh–Bénard on 16×16 tiles 10.9 instead of 11.8.
+//   - regions of 256 cells from 1025 groups on: that lattice on 8×8 tiles 8.8–9.2 instead of 9.5.
+//   - tiles with two steps per launch: 64² and 128² F32 cavities on 60×12 tiles 3.12 and 3.22 instead
+//     of 3.61 and 3.86, others within 1 %; the 56×8 tile in FP64: 700² 15.5 instead of 15.6.
 // Whether a step writes a second buffer instead of the one it reads, which saves one of its two
-// barriers: the 8×8 tile with 8 steps (83 KB in FP64, one group per CU, as many as its lattices
-// have), 128² BGK cavity F64 1.96 → 1.89, F32S 1.56 → 1.52 µs per step.  The other tiles also
-// serve lattices with several groups per CU, which lose more by the LDS (330² F32 on 16×16
-// tiles with 4 steps 3.9 → 4.5).
-constexpr bool tb2d_two_buffers(int TW, int TH, int K, bool thm) { return !thm && K == 8 && TW == 8 && TH == 8; }
+// barriers: the 8×8 tile with 8 steps where its groups have a CU each (83 KB in FP64): 128² BGK
+// cavity F64 1.96 → 1.89, F32S 1.56 → 1.52 µs per step.  Groups that share a CU lose more by the
+// LDS (330² F32 on 16×16 tiles with 4 steps 3.9 → 4.5).
+constexpr bool tb2d_two_buffers(int TW, int TH, int K, bool thm, bool late) {
+  return !thm && !late && K == 8 && TW == 8 && TH == 8;
+}
+// Waves per SIMD the register budget is set for.
+template <class R, int COLL, int TW, int TH, int K, bool THM, bool LATE>
+constexpr int tb2d_waves() {
+  constexpr int NE = (TW + 2 * K) * (TH + 2 * K);
+  if (tb2d_two_buffers(TW, TH, K, THM, LATE)) return 3;
+  if (LATE && NE < 1024 && sizeof(R) == 4) return THM ? 5 : 7;
+  if (LATE && NE == 576 && COLL != KMI_BGK) return 5;
+  return 4;
+}
 
-template <int ST, int COLL, int TW, int TH, int K, bool THM>
-__global__ void __launch_bounds__((TW + 2 * K) * (TH + 2 * K), tb2d_two_buffers(TW, TH, K, THM) ? 3 : 4)
+template <int ST, int COLL, int TW, int TH, int K, bool THM, bool LATE>
+__global__ void __launch_bounds__((TW + 2 * K) * (TH + 2 * K),
+                                  (tb2d_waves<typename Store<ST>::real, COLL, TW, TH, K, THM, LATE>()))
     k_step_tb2d(const StepArgs a) {
   using S = Store<ST>;
   using E = typename S::elem;
@@ -49,7 +70,7 @@ __global__ void __launch_bounds__((TW + 2 * K) * (TH + 2 * K), tb2d_two_buffers(
   constexpr bool SH = S::shifted;
   constexpr int EW = TW + 2 * K, EH = TH + 2 * K, NE = EW * EH;
   constexpr bool DEAL = sizeof(R) == 8;
-  constexpr bool TWOBUF = tb2d_two_buffers(TW, TH, K, THM);
+  constexpr bool TWOBUF = tb2d_two_buffers(TW, TH, K, THM, LATE);
   constexpr int NV = (THM ? 18 : 9) * NE;
   __shared__ R lds[(TWOBUF ? 2 : 1) * NV];
   R* L = lds;
@@ -81,6 +102,16 @@ __global__ void __launch_bounds__((TW + 2 * K) * (TH + 2 * K), tb2d_two_buffers(
   __syncthreads();
 
   R nv[9], gv[9];
+  // the tile's own cells: step t+K straight from registers
+  auto store = [&](int ux, int uy) {
+    if (ux >= nx || uy >= ny) return;
+    const long long self = ux + (long long)nx * uy;
+    sfor<9>([&](auto qc) {
+      constexpr int q = decltype(qc)::value;
+      S::template st<false>(fo, self + q * P, nv[q]);
+      if constexpr (THM) GS::template st<false>(go, self + q * P, gv[q]);
+    });
+  };
   for (int s = 1; s <= K; ++s) {
     int ex = tid % EW, ey = tid / EW;
     if constexpr (DEAL) {
@@ -199,15 +230,8 @@ __global__ void __launch_bounds__((TW + 2 * K) * (TH + 2 * K), tb2d_two_buffers(
       });
     }
     if (s == K) {
-      // the tile's own cells: step t+K straight from registers
-      if (active && ux < nx && uy < ny) {
-        const long long self = ux + (long long)nx * uy;
-        sfor<9>([&](auto qc) {
-          constexpr int q = decltype(qc)::value;
-          S::template st<false>(fo, self + q * P, nv[q]);
-          if constexpr (THM) GS::template st<false>(go, self + q * P, gv[q]);
-        });
-      }
+      if constexpr (!LATE)
+        if (active) store(ux, uy);
       break;
     }
     if constexpr (TWOBUF) {
@@ -223,6 +247,11 @@ __global__ void __launch_bounds__((TW + 2 * K) * (TH + 2 * K), tb2d_two_buffers(
         if constexpr (THM) G[q * NE + e] = storage_round<thermal_storage(ST)>(gv[q]);
       });
     __syncthreads();
+  }
+  if constexpr (LATE) {
+    int ix = tid % EW - K, iy = tid / EW - K;
+    if constexpr (DEAL) ix = tid % TW, iy = tid / TW;
+    if (ix >= 0 && ix < TW && iy >= 0 && iy < TH) store(ox + K + ix, oy + K + iy);
   }
 }
 
@@ -245,20 +274,33 @@ bool tb2d_variant(int tile, int& TW, int& TH, int& K) {
   }
 }
 
-template <int ST, int COLL, int TW, int TH, int K>
-static hipError_t launch_tb(const StepArgs& a, bool th, hipStream_t s) {
-  const dim3 g(unsigned((a.nx + TW - 1) / TW), unsigned((a.ny + TH - 1) / TH)), b((TW + 2 * K) * (TH + 2 * K));
+template <int ST, int COLL, int TW, int TH, int K, bool LATE>
+static hipError_t launch_tb_groups(const StepArgs& a, bool th, dim3 g, hipStream_t s) {
+  const dim3 b((TW + 2 * K) * (TH + 2 * K));
   if (th) {
     // the thermal chain collides f with Guo BGK; FP64 f and g exceed the registers of a
     // 1024-wide group, so FP64 thermal lattices keep single-step launches
     if constexpr (COLL == KMI_BGK && ST != KMI_STORE_F64)
-      hipLaunchKernelGGL((k_step_tb2d<ST, COLL, TW, TH, K, true>), g, b, 0, s, a);
+      hipLaunchKernelGGL((k_step_tb2d<ST, COLL, TW, TH, K, true, LATE>), g, b, 0, s, a);
     else
       return hipErrorInvalidValue;
   } else {
-    hipLaunchKernelGGL((k_step_tb2d<ST, COLL, TW, TH, K, false>), g, b, 0, s, a);
+    hipLaunchKernelGGL((k_step_tb2d<ST, COLL, TW, TH, K, false, LATE>), g, b, 0, s, a);
   }
   return hipGetLastError();
+}
+
+template <int ST, int COLL, int TW, int TH, int K>
+static hipError_t launch_tb(const StepArgs& a, bool th, hipStream_t s) {
+  const dim3 g(unsigned((a.nx + TW - 1) / TW), unsigned((a.ny + TH - 1) / TH));
+  constexpr int NE = (TW + 2 * K) * (TH + 2 * K);
+  if constexpr (K == 2 || (TW == 56 && ST == KMI_STORE_F64)) {
+    return launch_tb_groups<ST, COLL, TW, TH, K, true>(a, th, g, s);
+  } else {
+    if constexpr (NE < 1024)
+      if ((long long)g.x * g.y > (NE == 576 ? 256 : 1024)) return launch_tb_groups<ST, COLL, TW, TH, K, true>(a, th, g, s);
+    return launch_tb_groups<ST, COLL, TW, TH, K, false>(a, th, g, s);
+  }
 }
 
 template <int ST, int COLL>
