@@ -314,13 +314,21 @@ static hipError_t launch(bool nts, const StepArgs& a, dim3 g, dim3 b, hipStream_
     if (b.x % 64 == 0) {
       // Work-groups run on XCD (linear index) mod 8.  Rows that follow each other share cache
       // lines where the row length is no multiple of a line, so each XCD takes a band of them
-      // (cavity 100³ F32S 30.5 → 26.4 µs a step, sphere 180×90×90 F32 49.5 → 44.0, 128³ F64
-      // whose rows are whole lines 130 → 133).
+      // (cavity 100³ F32S 30.5 → 26.4 µs a step, sphere 180×90×90 F32 49.5 → 44.0).  The bands
+      // need a multiple of 8 rows of groups, and the XCDs that hold the rows added idle: worth it
+      // while those are fewer bytes than what the others share, some 80 of a row's (walled boxes
+      // F64, µs a step with bands / without: 150×60×166 105 / 109, 65×17×1000 99 / 81, 65×9×2000
+      // 130 / 89), and on rows of up to 10 KB (D2Q9 F32 2050² 62 / 64.6, F64 2050² 133 / 127).
+      // D2Q9 lattices whose two buffers stay in the L2s (32 MB) take bands of any padding and
+      // length: each XCD reads the rows it wrote a step ago (F64 5000×17 4.8 / 5.8, 20000×9 7.5 / 9.3).
       StepArgs r = a;
       r.xcd_shift = 0;
-      if (g.y < 65528u) {
+      const unsigned gy = (g.y + 7u) / 8u * 8u;
+      const double row = double(a.nx) * sizeof(typename Store<ST>::elem);
+      const bool resident = Q == 9 && 18.0 * row * a.ny <= 32e6;
+      if (gy < 65536u && (resident || (row <= 10e3 && double(gy - g.y) * row <= 80.0 * g.y))) {
         r.xcd_shift = g.x % 8 == 0 ? 0 : g.x % 4 == 0 ? 1 : g.x % 2 == 0 ? 2 : 3;
-        g.y = (g.y + 7u) / 8u * 8u;
+        g.y = gy;
       }
       if (nts) hipLaunchKernelGGL((k_step<Q, ST, COLL, TH, BND, true, true>), g, b, 0, s, r);
       else hipLaunchKernelGGL((k_step<Q, ST, COLL, TH, BND, false, true>), g, b, 0, s, r);
