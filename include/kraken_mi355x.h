@@ -439,9 +439,10 @@ int kmi_batch_set_launch(kmi_batch* b, int32_t tw, int32_t th, int32_t groups, i
 int kmi_batch_get_launch(const kmi_batch* b, int32_t* tw, int32_t* th, int32_t* groups,
                          int32_t* nontemporal);
 /* Steps per launch: 1; 2 (the tile's step t+1, with a one-cell ring, kept in LDS; HBM
- * sees one read and one write per population per two steps); 3 or 4 (strips of columns
- * marched up the cavities, the intermediate steps in registers; tiles of width 16, 32 or 64,
- * which the residual sums keep using).  Bit-identical to single steps; step counts that are not a multiple end
+ * sees one read and one write per population per two steps); 3 or 4 (tiles of width 16, 32 or
+ * 64: batches of few tiles advance the tile and a 3- or 4-cell ring in LDS, others march strips
+ * of columns up the cavities, the intermediate steps in registers; the running cavities' number
+ * of tiles decides, and the residual sums use the tiles).  Bit-identical to single steps; step counts that are not a multiple end
  * with two-step and single-step launches.  Chosen by kmi_batch_autotune. */
 int kmi_batch_set_temporal(kmi_batch* b, int32_t steps_per_launch);
 int kmi_batch_get_temporal(const kmi_batch* b, int32_t* steps_per_launch);

@@ -182,12 +182,82 @@ __global__ void __launch_bounds__(256) k_batch_step2(const BatchArgs a) {
   }
 }
 
-// K steps per launch (K = 3 or 4): the register march of kmi_march2d.h, one wave per piece
-// (cavity, columns [x0, x1), rows [y0, y1)) of a table the host lays out (batch_build_pieces).
-// Bit-identical to K single steps.  256 cavities of 64–512 cells a side, F32S MRT: 172 (K = 3)
-// and 221 GLUPS (K = 4) where a kernel that advanced each tile and its K-cell ring in LDS ran
-// 122 and 117; 256 of 128²: 167 and 204 against 129 and 119.  The two-step tile kernel above
-// (124 and 114 GLUPS) stays for two steps: marching K = 2 levels runs 89–121.
+// K steps per launch (K = 3 or 4) over the same tile slots: the tile and a K-cell ring are
+// loaded into LDS with one work-item per cell of that region ((tw+2K)(th+2K) ≤ 1024), then
+// advanced K steps in place (step s updates the region less s cells on each side: read,
+// barrier, write back in the storage rounding, barrier); the tile's t+K populations go to
+// HBM.  Bit-identical to K single steps.  Dynamic LDS: 9 · (tw+2K)(th+2K) reals.  For batches of
+// few tiles (stepK_lds): bound by one region's chain of K dependent steps.
+template <int ST, int COLL, int K>
+__global__ void __launch_bounds__(1024) k_batch_stepK(const BatchArgs a) {
+  using S = Store<ST>;
+  using E = typename S::elem;
+  using R = typename S::real;
+  R* const L = reinterpret_cast<R*>(kmi_batch_lds);
+  const int tw = a.tw, th = 256 / a.tw;
+  const int ew = tw + 2 * K, eh = th + 2 * K, ne = ew * eh;
+  const int e = threadIdx.x;  // one work-item per region cell (blockDim.x == ne)
+  const int ex = e % ew, ey = e / ew;
+  for (int t = blockIdx.x; t < a.nslots; t += gridDim.x) {
+    const int c = a.slots[3 * t];  // uniform over the work-group
+    if (c < 0) continue;
+    const CavRec cv = a.cav[c];
+    const int n = cv.n;
+    const int i = a.slots[3 * t + 1] - K + ex, j = a.slots[3 * t + 2] - K + ey;
+    const bool in = i >= 0 && j >= 0 && i < n && j < n;
+    const unsigned P = unsigned(n) * unsigned(n);
+    const E* __restrict__ src = static_cast<const E*>(a.fi) + cv.foff;
+    E* __restrict__ dst = static_cast<E*>(a.fo) + cv.foff;
+    if (in) {
+      const unsigned self = unsigned(i + n * j);
+      sfor<9>([&](auto qc) {
+        constexpr int q = decltype(qc)::value;
+        L[q * ne + e] = S::ld(src, self + unsigned(q) * P);
+      });
+    }
+    __syncthreads();
+    R fr[9];
+    for (int s = 1; s <= K; ++s) {
+      const bool valid = in && ex >= s && ex < ew - s && ey >= s && ey < eh - s;
+      if (valid) {
+        R fp[9];
+        cavity_pull(a, n, i, j, unsigned(e), unsigned(ew), unsigned(ne), fp,
+                    [&](unsigned off) { return L[off]; });
+        cavity_collide<ST, COLL>(a, cv, n, j, fp, fr);
+      }
+      if (s == K) break;
+      __syncthreads();  // every step-s read of L is done
+      if (valid) {
+        sfor<9>([&](auto qc) {
+          constexpr int q = decltype(qc)::value;
+          L[q * ne + e] = storage_round<ST>(fr[q]);
+        });
+      }
+      __syncthreads();
+    }
+    if (in && ex >= K && ex < K + tw && ey >= K && ey < K + th) {
+      const unsigned self = unsigned(i + n * j);
+      sfor<9>([&](auto qc) {
+        constexpr int q = decltype(qc)::value;
+        S::template st<false>(dst, self + unsigned(q) * P, fr[q]);
+      });
+    }
+    __syncthreads();  // the next slot's load overwrites LDS
+  }
+}
+
+// Work-items of a K-step region for tile width tw (0: the region exceeds 1024).
+KMI_HD int stepK_region(int tw, int K) {
+  const int r = (tw + 2 * K) * (256 / tw + 2 * K);
+  return r <= 1024 ? r : 0;
+}
+
+// K steps per launch (K = 3 or 4) of batches with many tiles: the register march of
+// kmi_march2d.h, one wave per piece (cavity, columns [x0, x1), rows [y0, y1)) of a table the host
+// lays out (batch_build_pieces).  Bit-identical to K single steps.  256 cavities of 64–512 cells
+// a side, F32S MRT: 172 (K = 3) and 221 GLUPS (K = 4) where the LDS kernel above runs 122 and 117;
+// 256 of 128²: 167 and 204 against 129 and 119.  The two-step tile kernel (124 and 114 GLUPS)
+// stays for two steps: marching K = 2 levels runs 89–121.
 struct MarchPiece {
   int cav;        // −1: padding
   int x0x1, y0y1;  // first and one past the last column / row, 16 bits each
@@ -237,8 +307,18 @@ __global__ void __launch_bounds__(256, (march_waves<ST, K>()))
   else march2d<ST, K, true>(d, xs, xe, y0, y1);
 }
 
-// Tile widths that 3 or 4 steps per launch take (the tiles still carry the residual).
-static bool stepK_tile(int tw, int K) { return (tw + 2 * K) * (256 / tw + 2 * K) <= 1024; }
+// Whether 3 or 4 steps per launch run on the LDS tiles: up to the number of tile slots at which the
+// march, which needs a wave for every few rows of a strip and evaluates at least 4 + 3 rows in turn,
+// catches up.  µs per step, LDS / march: F32S MRT, four steps, 64×4 tiles: one 64² cavity 1.45 /
+// 3.20, 32 (512 slots) 1.92 / 3.33, 64 3.97 / 3.51; on 16×16 tiles 128 cavities of 64² (2,048
+// slots) 5.05 / 4.84; F64 BGK, 64×4, 32 cavities of 64² 3.5 / 4.2, 64 6.7 / 4.8.
+static bool stepK_lds(int st, int tw, int K, int slots) {
+  static const int limit[3][2][3] = {{{1024, 768, 512}, {768, 768, 512}},      // FP64: 3, 4 steps on width 16, 32, 64
+                                     {{4096, 1024, 1024}, {1280, 1024, 640}},  // FP32
+                                     {{4096, 1792, 1152}, {2304, 1792, 960}}};  // F32S, F16S
+  const int kind = st == KMI_STORE_F64 ? 0 : st == KMI_STORE_F32 ? 1 : 2;
+  return slots <= limit[kind][K - 3][tw >= 64 ? 2 : tw >= 32 ? 1 : 0];
+}
 
 // Velocity of a cell from the stored populations, FP64 (compute_macroscopic_2d order).
 template <int ST>
@@ -430,6 +510,28 @@ static hipError_t launch_batch_step2(int st, int coll, bool nts, const BatchArgs
   return hipGetLastError();
 }
 
+static hipError_t launch_batch_stepK(int st, int coll, int K, const BatchArgs& a, int groups, hipStream_t s) {
+  const int ne = stepK_region(a.tw, K);
+  if (ne == 0) return hipErrorInvalidValue;
+  const dim3 g(static_cast<unsigned>(groups)), b(static_cast<unsigned>(ne));
+#define KMI_BATCH_COLLK(ST)                                                                      \
+  {                                                                                             \
+    const size_t sh = size_t(9) * ne * sizeof(typename Store<ST>::real);                        \
+    if (K == 3) {                                                                               \
+      if (coll == KMI_BGK) hipLaunchKernelGGL((k_batch_stepK<ST, KMI_BGK, 3>), g, b, sh, s, a); \
+      else if (coll == KMI_TRT) hipLaunchKernelGGL((k_batch_stepK<ST, KMI_TRT, 3>), g, b, sh, s, a); \
+      else hipLaunchKernelGGL((k_batch_stepK<ST, KMI_MRT, 3>), g, b, sh, s, a);                 \
+    } else {                                                                                    \
+      if (coll == KMI_BGK) hipLaunchKernelGGL((k_batch_stepK<ST, KMI_BGK, 4>), g, b, sh, s, a); \
+      else if (coll == KMI_TRT) hipLaunchKernelGGL((k_batch_stepK<ST, KMI_TRT, 4>), g, b, sh, s, a); \
+      else hipLaunchKernelGGL((k_batch_stepK<ST, KMI_MRT, 4>), g, b, sh, s, a);                 \
+    }                                                                                           \
+  }
+  KMI_BATCH_ST(st, KMI_BATCH_COLLK(ST));
+#undef KMI_BATCH_COLLK
+  return hipGetLastError();
+}
+
 static hipError_t launch_batch_march(int st, int coll, int K, const BatchArgs& a, const MarchPiece* pieces,
                                      int npieces, hipStream_t s) {
   const dim3 g(static_cast<unsigned>(npieces / 4)), b(256);
@@ -480,7 +582,8 @@ struct kmi_batch {
   int cur = 0;
   // tiles
   int tw = 64, th = 4, groups = 0, nts = 0;
-  int span = 1;  // steps per launch: 1, 2 (k_batch_step2), 3 or 4 (k_batch_march)
+  int span = 1;  // steps per launch: 1, 2 (k_batch_step2), 3 or 4 (k_batch_stepK, k_batch_march)
+  bool lds = false;  // span 3 or 4: k_batch_stepK on the tile slots
   bool tiles_dirty = true;
   int nslots = 0;
   int* slots_d = nullptr;
@@ -527,7 +630,7 @@ static int batch_groups(const kmi_batch* B) {
 static void batch_build_pieces(kmi_batch* B, std::vector<MarchPiece>& out) {
   out.clear();
   B->npieces = 0;
-  if (B->span < 3) return;
+  if (B->span < 3 || B->lds) return;
   std::vector<std::pair<int, int>> sides;  // (side, running cavities)
   for (int cv = 0; cv < B->ncav; ++cv) {
     if (B->status[cv] != KMI_CAV_RUNNING) continue;
@@ -619,6 +722,7 @@ static int batch_build_tiles(kmi_batch* B) {
   KMI_HIP(c, grow((void**)&B->slots_d, B->slots_cap, slots.size() * sizeof(int)));
   KMI_HIP(c, grow((void**)&B->cav_slots_d, B->cav_slots_cap, cav_slots.size() * sizeof(int)));
   KMI_HIP(c, grow((void**)&B->partials, B->partials_cap, size_t(4) * B->nslots * sizeof(double)));
+  B->lds = B->span >= 3 && stepK_lds(B->desc.storage, B->tw, B->span, B->nslots);
   std::vector<MarchPiece> pieces;
   batch_build_pieces(B, pieces);
   if (!pieces.empty()) {
@@ -671,10 +775,11 @@ static int batch_launch_step2(kmi_batch* B, hipStream_t s) {
   return KMI_OK;
 }
 
-static int batch_launch_march(kmi_batch* B, hipStream_t s) {
+static int batch_launch_multi(kmi_batch* B, hipStream_t s) {
   BatchArgs a = batch_args(B);
   hipError_t e =
-      launch_batch_march(B->desc.storage, B->desc.collision, B->span, a, B->pieces_d, B->npieces, s);
+      B->lds ? launch_batch_stepK(B->desc.storage, B->desc.collision, B->span, a, batch_groups(B), s)
+             : launch_batch_march(B->desc.storage, B->desc.collision, B->span, a, B->pieces_d, B->npieces, s);
   if (e != hipSuccess) return hip_fail(B->ctx, e, "batch multi-step launch");
   B->cur ^= 1;
   return KMI_OK;
@@ -684,7 +789,7 @@ static int batch_launch_march(kmi_batch* B, hipStream_t s) {
 static int batch_launch_n(kmi_batch* B, int64_t n, hipStream_t s) {
   if (B->span >= 3)
     for (; n >= B->span; n -= B->span)
-      if (int rc = batch_launch_march(B, s)) return rc;
+      if (int rc = batch_launch_multi(B, s)) return rc;
   if (B->span >= 2)
     for (; n >= 2; n -= 2)
       if (int rc = batch_launch_step2(B, s)) return rc;
@@ -1084,7 +1189,7 @@ int kmi_batch_set_launch(kmi_batch* B, int32_t tw, int32_t th, int32_t groups, i
   if (!B) return fail(nullptr, KMI_ERR_ARG, "batch is NULL");
   if (!((tw == 16 || tw == 32 || tw == 64 || tw == 128 || tw == 256) && tw * th == 256) || groups < 0)
     return fail(B->ctx, KMI_ERR_ARG, "kmi_batch_set_launch: tiles of tw x th = 256 cells, tw in {16,32,64,128,256}");
-  if (B->span >= 3 && !stepK_tile(tw, B->span))
+  if (B->span >= 3 && stepK_region(tw, B->span) == 0)
     return fail(B->ctx, KMI_ERR_ARG, "kmi_batch_set_launch: tile too wide for the current steps per launch");
   KMI_HIP(B->ctx, hipSetDevice(B->ctx->device));
   KMI_HIP(B->ctx, hipStreamSynchronize(B->ctx->stream));
@@ -1101,7 +1206,7 @@ int kmi_batch_set_temporal(kmi_batch* B, int32_t steps_per_launch) {
   if (!B) return fail(nullptr, KMI_ERR_ARG, "batch is NULL");
   if (steps_per_launch < 1 || steps_per_launch > 4)
     return fail(B->ctx, KMI_ERR_ARG, "kmi_batch_set_temporal: steps per launch must be 1, 2, 3 or 4");
-  if (steps_per_launch >= 3 && !stepK_tile(B->tw, steps_per_launch))
+  if (steps_per_launch >= 3 && stepK_region(B->tw, steps_per_launch) == 0)
     return fail(B->ctx, KMI_ERR_ARG,
                 "kmi_batch_set_temporal: 3 or 4 steps per launch need tiles of width 16, 32 or 64");
   KMI_HIP(B->ctx, hipSetDevice(B->ctx->device));
@@ -1152,10 +1257,11 @@ int kmi_batch_autotune(kmi_batch* B, int64_t steps_per_trial, double* best_ms) {
         B->groups = g;
         B->nts = nt & 1;
         B->span = 1 + (nt >> 1);
-        // the register march depends on neither tile, groups nor store policy: timed once
-        if (B->span >= 3 && (B->nts || g != 0 || B->tw != 64)) continue;
+        if (B->span >= 3 && (B->nts || stepK_region(B->tw, B->span) == 0)) continue;  // their stores are plain
         if (batch_build_tiles(B) != KMI_OK) { e = hipErrorUnknown; break; }
         if (g > 0 && g >= B->nslots) continue;  // same as one group per slot
+        // the register march depends on neither tile nor groups: timed once
+        if (B->span >= 3 && !B->lds && (g != 0 || B->tw != 64)) continue;
         if (batch_launch_n(B, B->span, x->stream) != KMI_OK) { e = hipErrorUnknown; break; }
         double t = 1e300;
         for (int rep = 0; rep < 2 && e == hipSuccess; ++rep) {

@@ -145,8 +145,9 @@ class Batch:
 
     def set_temporal(self, steps_per_launch):
         """1: one step per launch; 2: two steps per launch (step t+1 of each tile and its ring
-        kept in LDS); 3 or 4: strips of columns marched up the cavities in registers (tile
-        width 16, 32 or 64, which the residual sums use).  Bit-identical to single steps."""
+        kept in LDS); 3 or 4 (tile width 16, 32 or 64): the tile and a 3- or 4-cell ring advanced
+        in LDS where the running cavities have few tiles, else strips of columns marched up the
+        cavities in registers.  Bit-identical to single steps."""
         self._chk(L.load().kmi_batch_set_temporal(self._h, int(steps_per_launch)))
 
     def autotune(self, steps_per_trial=8):
