@@ -354,8 +354,9 @@ int kmi_lattice_get_launch(const kmi_lattice* lat, int32_t* bx, int32_t* by, int
  * plus its ring on each axis, zchunks 1; the tile and a ring of as many cells as steps are
  * advanced in LDS, one work-item per cell: 1 = 28x28 two steps, 2 = 24x24 four, 3 = 56x8
  * four, 4 = 16x16 eight, 5 = 60x12 two, 6 = 8x8 four, 7 = 16x16 four, 8 = 8x8 eight.  Tile 2
- * of a lattice of at least 160,000 cells without mask, forcing or thermal populations marches
- * strips of columns in registers instead (four steps as well).
+ * of a lattice without mask, forcing or thermal populations marches strips of columns in
+ * registers instead (four steps as well) where that is the faster one: from 160,000 cells on, by
+ * storage and shape.
  * Results are bit-identical to single-step launches; step counts that are not a multiple
  * of the span end with single steps.
  * A D3Q19 lattice on which no launch was set (here, by kmi_lattice_set_launch or by

@@ -442,13 +442,10 @@ static bool tb_eligible(const kmi_lattice* L, int tile, bool any_extent = false)
 }
 
 // Whether tile 2 (24×24, four steps) of a D2Q9 lattice runs the register march
-// (kmi_march2d.hip): no thermal populations, mask or forcing, and at least 160,000 cells.
-// Below that the march has too few waves (µs per step, tile / march, F64 periodic: 320² 4.4 /
-// 4.5, 400² 6.9 / 4.6, 512² 8.1 / 5.6, 2048² 90 / 40; F32S cavity: 320² 3.3 / 5.0, 400² 5.2 /
-// 5.0, 640² 7.6 / 6.2, 2048² 61 / 23).
+// (kmi_march2d.hip): no thermal populations, mask or forcing, and sizes at which it is faster.
 static bool march_applies(const kmi_lattice* L) {
   return L->Q == 9 && L->tb_tile == 2 && !L->desc.thermal && !L->mask && L->desc.forcing == KMI_FORCE_NONE &&
-         L->ncells >= 160000;
+         march2d_wins(L->desc.storage, L->desc.collision, L->args);
 }
 
 // Steps advanced by one launch.

@@ -63,7 +63,9 @@ hipError_t launch_step2(int st, int coll, int tile, int zchunks, bool nts, bool 
 // (tb2d_variant).
 bool tb2d_variant(int tile, int& TW, int& TH, int& K);
 hipError_t launch_step_tb2d(int st, int coll, int tile, bool th, const StepArgs& a, hipStream_t s);
-// Four steps per launch on a large D2Q9 lattice (kmi_march2d.hip).
+// Four steps per launch on a large D2Q9 lattice (kmi_march2d.hip); march2d_wins: faster there than
+// the LDS tile of four steps.
+bool march2d_wins(int st, int coll, const StepArgs& a);
 hipError_t launch_march2d(int st, int coll, const StepArgs& a, hipStream_t s);
 hipError_t launch_copy_probe(const void* src, void* dst, long long bytes, hipStream_t s);
 hipError_t launch_to_storage(int Q, int st, const double* src, void* dst, long long ncells,

@@ -104,6 +104,35 @@ static hipError_t launch_march_st(int coll, const StepArgs& a, hipStream_t s) {
   return launch_march_coll<ST, KMI_BGK>(a, s);
 }
 
+// Where the march beats the 24×24 tile with four steps (k_step_tb2d).  The tile's time hardly grows up
+// to 512 work-groups, two to a CU (FP64: one, 256), while a march that short of rows is bound by the
+// 4 + 3 and more rows each wave evaluates in turn.  What moves the line, µs per step, tile / march:
+//   - strips whose lanes are half empty between walls (channel 70×5714 F64 BGK 11.9 / 14.2): 0.7 of the groups;
+//   - x faces with a closure or a Ladd term, whose tests sit in the row loop (channel F32S MRT 500² 5.6 /
+//     7.5, 1024² 17.2 / 15.8, 1200² 21.7 / 19.4; F64 BGK 700² 14.6 / 11.8);
+//   - F16S, whose conversions the tile hides better (BGK cavity 500² 5.4 / 6.5, 700² 9.0 / 7.6);
+//   - within the tile's first round (FP64: second) the march needs, between x walls, filled strips of
+//     some rows (F32 BGK box 400² 5.2 / 4.2, periodic 400² 5.2 / 3.9), and in FP32 y faces without
+//     closures or Ladd terms (F32 MRT cavity 500² 5.8 / 6.2).
+// Over 4,142 lattices of 165,000–4,200,000 cells (every storage; BGK, MRT; periodic, walls, lids,
+// channels; squares, 32–240 wide, 32–200 high): always marching 0.862 of the tile's time and up to
+// 1.8, this rule 0.827 and up to 1.16, the better of both 0.821.
+bool march2d_wins(int st, int coll, const StepArgs& a) {
+  if ((long long)a.nx * a.ny < 160000) return false;
+  const bool f64 = st == KMI_STORE_F64, f16 = st == KMI_STORE_F16S, perx = a.per[0] != 0;
+  const bool restx = rests(a.face[KMI_WEST].kind) && rests(a.face[KMI_EAST].kind);
+  const bool resty = rests(a.face[KMI_SOUTH].kind) && rests(a.face[KMI_NORTH].kind);
+  const bool filled = 10LL * a.nx >= 6LL * 64 * march_strips(a.nx, 4, perx).m;
+  long long groups = (long long)((a.nx + 23) / 24) * ((a.ny + 23) / 24);
+  if (!perx && !filled && !(f64 && restx)) groups = groups * 7 / 10;
+  if (!restx) return groups > (f64 ? 840 : f16 ? 2200 : 1800);
+  if (f16) return groups > (perx ? 512 : 840);
+  if (groups > 512) return true;
+  const bool snug = a.ny >= 64 && a.nx >= 56 && filled;
+  if (perx) return snug || st != KMI_STORE_F32 || coll != KMI_MRT;
+  return snug && (f64 || resty);
+}
+
 hipError_t launch_march2d(int st, int coll, const StepArgs& a, hipStream_t s) {
   switch (st) {
     case KMI_STORE_F64: return launch_march_st<KMI_STORE_F64>(coll, a, s);

@@ -291,7 +291,7 @@ class Lattice:
         12: 64×8, 13: 32×16, 14: 32×8 with a thread per cell of the tile and its ring) or three (6: 64×8, 7: 32×8,
         8: 32×16 with a thread per cell; 9: 32×8, 10: 32×16, 11: 64×8 with a thread per cell
         of the tile and its two-cell ring; FP64 only 7 and 9).  D2Q9 lattice without thermal populations, cut links or
-        per-node faces: 1: 28×28 two steps, 2: 24×24 four (lattices of 160,000 cells and more
+        per-node faces: 1: 28×28 two steps, 2: 24×24 four (large lattices
         without mask, forcing or thermal populations: strips marched in registers), 3: 56×8 four, 4: 16×16 eight,
         5: 60×12 two, 6: 8×8 four, 7: 16×16 four, 8: 8×8 eight.  0: off.  Bit-identical to single steps.
         A D3Q19 lattice on which neither this nor set_launch nor autotune was called picks its own
