@@ -28,9 +28,10 @@ constexpr int kRedPartials = kRedGroups * 3 * 2;  // groups × 3 values × (sum,
 int fail(kmi_ctx* ctx, int code, const std::string& msg);
 int hip_fail(kmi_ctx* ctx, hipError_t e, const char* what);
 
-// Host transfers on ctx->stream through the context's pinned buffers (kmi_xfer.hip).
-// copy_to_host returns when the data has arrived (and with it everything queued before);
-// copy_to_device when the host arrays may change, the device side in stream order.
+// Host transfers on ctx->stream (kmi_xfer.hip), through the context's pinned buffers where that
+// is faster.  copy_to_host returns when the data has arrived (and with it everything queued
+// before); copy_to_device is in stream order, and the host arrays may change once the stream has
+// been waited for.
 struct HostSeg {
   void* host;
   void* dev;
