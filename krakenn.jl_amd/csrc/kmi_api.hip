@@ -1065,6 +1065,7 @@ static MomForce mom_force(const kmi_lattice* L) {
 
 static int reduce_cells(kmi_lattice* L, int kind, double* out3) {
   kmi_ctx* c = L->ctx;
+  std::lock_guard<std::mutex> one(c->reducing);
   hipError_t e = launch_reduce_cells(L->Q, L->desc.storage, L->f[L->cur],
                                      L->desc.thermal ? L->g[L->cur] : nullptr, L->mask, L->uprev,
                                      L->ncells, L->plane, L->desc.T_ref, mom_force(L), kind,
@@ -1189,6 +1190,7 @@ int kmi_reduce(kmi_lattice* L, int32_t kind, int32_t arg, double* out) {
       if (hi1 - lo1 < 1 || hi2 - lo2 < 1 || n[ax] < 2)
         return fail(c, KMI_ERR_STATE, "kmi_reduce: grid too small for the Nusselt estimator");
       const double Th = d.faces[arg].T, dT = d.faces[arg].T - d.faces[opp].T;
+      std::lock_guard<std::mutex> one(c->reducing);
       hipError_t e = launch_nusselt(L->Q, d.storage, L->g[L->cur], int(d.nx), int(d.ny),
                                     int(n[2]), L->plane, d.T_ref, arg, Th, dT, lo1, hi1, lo2, hi2,
                                     c->partials, c->out, c->stream);
@@ -1202,6 +1204,7 @@ int kmi_reduce(kmi_lattice* L, int32_t kind, int32_t arg, double* out) {
     case KMI_RED_DRAG_HALFWAY: {
       if (L->nlinks > 0) {
         const kmi_desc& d = L->desc;
+        std::lock_guard<std::mutex> one(c->reducing);
         hipError_t e = launch_drag(L->Q, d.storage, L->f[L->cur], L->nlinks, L->link_cell,
                                    L->link_q, L->link_qw, L->link_uw, int(d.nx), int(d.ny),
                                    L->args.nz, L->plane, kind == KMI_RED_DRAG_MEA, c->partials,

@@ -1,6 +1,7 @@
 // kmi_internal.h — host-side internals shared by the C-ABI translation units.
 #pragma once
 
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -16,6 +17,7 @@ struct kmi_ctx {
   std::string err;
   double* partials = nullptr;  // kRedPartials values, then the reductions' group counter
   double* out = nullptr;       // 8 values in pinned host memory, written by the reductions
+  std::mutex reducing;         // held from a reduction's launch until its values are read
   kmi::HostCopier* copier = nullptr;
 };
 
