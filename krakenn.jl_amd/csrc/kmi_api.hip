@@ -103,8 +103,9 @@ int kmi_ctx_create(int device, kmi_ctx** out) {
   c->device = device;
   if ((e = hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking)) != hipSuccess ||
       (e = hipMalloc(&c->partials, (kRedPartials + 1) * sizeof(double))) != hipSuccess ||
-      (e = hipMemset(c->partials, 0, (kRedPartials + 1) * sizeof(double))) != hipSuccess ||
-      (e = hipDeviceSynchronize()) != hipSuccess ||
+      // on the context's own stream: other contexts may be running for long
+      (e = hipMemsetAsync(c->partials, 0, (kRedPartials + 1) * sizeof(double), c->stream)) != hipSuccess ||
+      (e = hipStreamSynchronize(c->stream)) != hipSuccess ||
       (e = hipHostMalloc(reinterpret_cast<void**>(&c->out), 8 * sizeof(double), hipHostMallocDefault)) != hipSuccess ||
       (e = resolve_noalloc_workspace(device)) != hipSuccess ||
       (e = (c->copier = host_copier_create()) ? hipSuccess : hipErrorOutOfMemory) != hipSuccess) {
