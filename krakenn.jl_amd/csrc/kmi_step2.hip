@@ -128,6 +128,18 @@ KMI_DEV void ladd_all(R (&f)[19], const StepArgs& a, const Nbr& n) {
   });
 }
 
+// A value the compiler may not carry over the planes of a march, in the general walled mode with
+// FP64 arithmetic.  There the pull's source offsets of every direction, the Ladd products of every
+// link and the constants of the Zou–He closures all count as loop constants and together need
+// more than the 256 registers a work-item has: without this 67–71 of them were spilled, and each
+// reload in the pull waits for the loads before it.  Working the offsets out again takes some
+// 100 integer instructions a plane beside 600 in FP64.
+template <int M, class R>
+KMI_DEV int per_plane(int v) {
+  if constexpr (M == 2 && sizeof(R) == 8) asm volatile("" : "+v"(v));
+  return v;
+}
+
 // Element at byte offset `off` of a population plane.  Plane bases are uniform (scalar
 // registers) and the offsets 32-bit, so each access is one saddr-form global instruction
 // with no 64-bit address arithmetic.  A field holds fewer than 2^31 / 19 cells, so every
@@ -219,7 +231,9 @@ KMI_DEV void update19(R (&fp)[19], R (&fo)[19], const StepArgs& a, int gx, int g
     constexpr bool SH = Store<ST>::shifted;
     for (int n = 0; n < a.n_zh; ++n) {
       const int fid = a.zh_face[n];
-      const FaceArgs& F = a.face[fid];
+      FaceArgs F = a.face[fid];
+      if constexpr (sizeof(R) == 8)
+        asm volatile("" : "+v"(F.rho), "+v"(F.u[0]), "+v"(F.u[1]), "+v"(F.u[2]));
       switch (fid) {
         case KMI_WEST: if (gx == 0) zh3_apply<SH, 0>(fp, F); break;
         case KMI_EAST: if (gx == a.nx - 1) zh3_apply<SH, 1>(fp, F); break;
@@ -468,7 +482,7 @@ KMI_DEV void march2_walled(const StepArgs& a, int zlen, int tx, int ty, int zc, 
     const int zm = tb::wrap(zs - 1, nz), zp = tb::wrap(zs + 1, nz);
 #pragma unroll
     for (int r = 0; r < EPT; ++r) {
-      const int e = tid + r * NT;
+      const int e = tb::per_plane<M, R>(tid + r * NT);
       if (e < NE && inside(s, e, mc)) {
         const int ex = e % EX, ey = e / EX;
         const int gx = tb::wrap(x0 - 1 + ex, nx), gy = tb::wrap(y0 - 1 + ey, ny);
@@ -514,7 +528,7 @@ KMI_DEV void march2_walled(const StepArgs& a, int zlen, int tx, int ty, int zc, 
     R keep0[EPT][9], keepp[EPT][5];
 #pragma unroll
     for (int r = 0; r < EPT; ++r) {
-      const int e = tid + r * NT;
+      const int e = tb::per_plane<M, R>(tid + r * NT);
       if (e < NE && inside(s, e, mc)) {
         R fn[19];
         const int gx = tb::wrap(x0 - 1 + e % EX, nx), gy = tb::wrap(y0 - 1 + e / EX, ny), gz = tb::wrap(s, nz);
@@ -537,7 +551,7 @@ KMI_DEV void march2_walled(const StepArgs& a, int zlen, int tx, int ty, int zc, 
       const R* const Br = B + ((u - 2) & 1) * 5 * NE;  // c_z = +1 of plane s−2
       const R* const Bo = B + ((u - 1) & 1) * 5 * NE;  // c_z = +1 of plane s−1 (own)
       const R* const Co = C + ((u - 1) & 1) * 5 * NE;  // c_z = −1 of plane s−1 (own)
-      const int ix = tid % TX, iy = tid / TX;
+      const int ti = tb::per_plane<M, R>(tid), ix = ti % TX, iy = ti / TX;
       const tb::Nbr nb = tb::nbr<M>(a, x0 + ix, y0 + iy, s - 1);
       R fp[19], fn[19];
       pull_lds<M>(fp, A, Br, Cw, Bo, Co, NE, EX, ix + 1, iy + 1, a, nb);
