@@ -10,10 +10,13 @@
 // and 64 − 2 (K − 1) columns are written (an edge on a wall needs no halo).  The rows above
 // and below a chunk of rows are evaluated again the same way.
 //
-// What bounds it: VALU issue for lattices in the last-level cache (F32S MRT, K = 4: 443
-// instructions per wave and iteration for 58 columns × 4 steps, against 405 for 256 cells ×
-// 2 steps plus their halo and two barriers in the tile kernel it replaced), HBM beyond it
-// (2048² F64: 36 B per cell update and 1.28 × that with the halos, 4.8 TB/s).  Why registers
+// What bounds it: the dependent loads and arithmetic of two waves per SIMD (the rows held take
+// the registers of more), near the rate of memory in FP64.  Counters of a 2048² BGK launch, four
+// steps: F64 154 µs for 360 MB read and 310 MB written (302 MB each without halos), 4.4 of the
+// 5.5 TB/s of a copy, the VALU busy 50 % of the time; a wave issues in 40 % of its cycles, waits
+// for its turn in 30 % and for a dependency in 30 %.  F32S: VALU busy 67 %, 53 / 17 / 30 %.
+// Instructions, F32S MRT, K = 4: 443 per wave and iteration for 58 columns × 4 steps, against 405
+// for 256 cells × 2 steps plus their halo and two barriers in the tile kernel.  Why registers
 // and not LDS: a tile of W × H cells with a K-cell ring in LDS evaluates (W + 2K)(H + 2K) / WH
 // cells (1.8 for 24×24, K = 4) and holds every wave at two barriers per step; a strip
 // evaluates 64/58 in x and (rows + 3)/rows in y, and no wave waits for another.
@@ -201,11 +204,6 @@ KMI_DEV void march2d(const Dom& d, int xs, int xe, int y0, int y1) {
         if constexpr (WX || GENERAL) d.template closures<GENERAL>(fp, gx, j);
         d.collide(fp, fo);
         if constexpr (l == K) {
-          // The row pulled ahead has to arrive before the stores are issued: the counter of
-          // outstanding accesses takes both in order, so a wait for these loads after the
-          // stores would be a wait for the stores as well.
-#pragma unroll
-          for (int q = 0; q < 9; ++q) ;
           if (mine) {
             const unsigned cell = unsigned(nx * j) * ES + ox[1];
             sfor<9>([&](auto qc) {

@@ -132,8 +132,11 @@ KMI_DEV void ladd_all(R (&f)[19], const StepArgs& a, const Nbr& n) {
 // FP64 arithmetic.  There the pull's source offsets of every direction, the Ladd products of every
 // link and the constants of the Zou–He closures all count as loop constants and together need
 // more than the 256 registers a work-item has: without this 67–71 of them were spilled, and each
-// reload in the pull waits for the loads before it.  Working the offsets out again takes some
-// 100 integer instructions a plane beside 600 in FP64.
+// reload in the pull waits for the loads before it (with the bounced links behind branches
+// 46–50, and loads that wait as well).  Working the offsets out again takes some 100 integer
+// instructions a plane beside 600 in FP64.  128³, tile 14 in 4 z-ranges, µs per step with the
+// spills / with branches / now: moving x wall 337 / 227 / 111, Zou–He x faces 312 / 216 / 119,
+// solid mask 390 / 241 / 122.
 template <int M, class R>
 KMI_DEV int per_plane(int v) {
   if constexpr (M == 2 && sizeof(R) == 8) asm volatile("" : "+v"(v));
@@ -1095,7 +1098,9 @@ static bool lean_walls(const StepArgs& a) {
   return true;
 }
 
-// The multi-step launch of a lattice whose user chose none.  A group marches zlen planes and
+// The multi-step launch of a lattice whose user chose none (with a solid mask: single steps; the
+// full walled variant is slower there, F32S 128³ 76 against 68 µs per step, or gains little,
+// F64 122 against 130).  A group marches zlen planes and
 // the planes its lower and upper levels need beyond them (two steps 2, three steps 4);
 // `per_cu` groups share a CU, and once every CU is taken the groups run in rounds, so a launch
 // takes rounds · (zlen + 2·(span − 1)) · plane, and the pair (tile, z-split) with the least
@@ -1131,7 +1136,8 @@ bool step2_plan(int st, bool bnd, const StepArgs& a, int& tile, int& zchunks) {
   const bool cached = bytes < 270e6;
   // a plane with Guo's source takes 1.34–1.45 times as long (F32 256×128×128 5.5 for 4.1 µs,
   // F64 6.95 for 4.8): ducts F32 200×110×100 76.8 / 67.6 µs per step, 256×128×128 128 / 93,
-  // F64 256×128×128 245 / 230; single steps for what stays in the cache (150×75×61 21.6 / 25.7)
+  // F64 256×128×128 245 / 230; in the cache the larger ones gain (F32 192×96×96 53.6 / 39.6) and
+  // the smaller keep single steps (150×75×61 21.6 / 25.7)
   const double force = a.forcing ? 1.45 : 1.0;
   double best = 0.95 * bytes / (cached ? 5.4e6 : a.nx * elem % 128 == 0 ? 5.3e6 : 4.5e6);
   for (const Cand& c : bnd ? walled[kind] : periodic[kind]) {
